@@ -112,33 +112,22 @@ const cplx<float>* agg_basis32(mgc_aggregation* a, hipStream_t s) {
   return a->basis32;
 }
 
-// Site mask of a block site: kind 0 = all, 1 = inner of point p, 2 = outer of
-// point p (outer for +mu: x_mu mod b = b-1; for -mu: x_mu mod b = 0).
-__device__ inline bool site_in_mask(const Lat4& blk, int xb, int kind, int p) {
-  if (kind == 0 || p == 8) return kind != 2;
-  int c[4];
-  blk.coords(xb, c);
-  const int mu = p & 3;
-  const bool outer = c[mu] == (p < 4 ? blk.L[mu] - 1 : 0);
-  return kind == 2 ? outer : !outer;
-}
-
 // ---------------------------------------------------------------------------
 // project: c(xc)(rhs)(k, i) = sum_{xb in mask, e in k} conj(U(xc,xb,e,i)) f(fine(xc,xb))(rhs)(e)
-// One workgroup per (coarse site, chunk of RC right-hand sides).  Thread
+// for one rhs (RCT = 1) or up to four (RCT = 4; wider calls: transfer_mfma.hip).
+// One workgroup per coarse site.  Thread
 // (i = t % nb, g = t / nb) walks rows q = g, g+G, ... of the block panel:
 // the nb threads of a group read one row's nb basis entries (contiguous) and
 // the G groups consecutive rows, so a wavefront streams the panel coalesced;
 // f(q) is a same-address broadcast load.  Group partial sums meet in LDS.
 // When the coarse lattice has few sites, blockIdx.z splits each panel into
 // gridDim.z row ranges of rows_per rows; the workgroups then write partial
-// sums to part[((xc * gridDim.y + y) * gridDim.z + z)][RC][2][nb], which
-// k_project_reduce adds in a fixed order.
+// sums to part[xc * gridDim.z + z][nrhs][2][nb], which k_project_reduce adds in a
+// fixed order.
 // With W = 2 (FP32, even nb) a thread takes the two adjacent basis columns
 // i = 2 i2, 2 i2 + 1 of each row in one 16-byte load, as the FP64 form reads
 // one column in 16 bytes; each column's sum keeps the row order q, q + G, ...
 // ---------------------------------------------------------------------------
-constexpr int RC = 4;  // right-hand sides per workgroup
 
 // W basis entries of one row from p (W = 2: FP32 only, p 16-byte aligned)
 template <typename R, int W>
@@ -153,19 +142,16 @@ __device__ __forceinline__ void project_row(const cplx<R>* p, cplx<R> (&o)[W]) {
   }
 }
 
-// RCT = right-hand sides a workgroup actually holds (1 for a single rhs)
-template <typename R, int RCT, int W = 1>
+template <typename R, int RCT, int W>
 __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
                                                  const cplx<R>* __restrict__ f,
                                                  cplx<R>* __restrict__ c,
                                                  const int* __restrict__ blk_fine, int nb, int Vb,
-                                                 int Ef, int nrhs, Lat4 blk, int kind, int point,
+                                                 int Ef, int nr, Lat4 blk, int kind, int point,
                                                  int rows_per, cplx<R>* __restrict__ part) {
   extern __shared__ unsigned char smem_raw[];
-  cplx<R>* s_red = reinterpret_cast<cplx<R>*>(smem_raw);  // [G][RC][2][nb]
+  cplx<R>* s_red = reinterpret_cast<cplx<R>*>(smem_raw);  // [G][RCT][2][nb]
   const int xc = blockIdx.x;
-  const int r0 = blockIdx.y * RC;
-  const int nr = min(RC, nrhs - r0);
   const int tid = threadIdx.x;
   const int nw = nb / W;  // threads per row
   const int G = blockDim.x / nw;
@@ -196,7 +182,7 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
           const int xb = qq / Ef, e = qq - xb * Ef;
           lo[v] = e < half;
           project_row<R, W>(Ub + (size_t)qq * nb + i, uu[v]);
-          fp[v] = f + ((size_t)bf[xb] * nrhs + r0) * Ef + e;
+          fp[v] = f + (size_t)bf[xb] * nr * Ef + e;
         }
         cplx<R> xv[PU][RCT];
 #pragma unroll
@@ -221,7 +207,7 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
       const int k = e >= half;
       cplx<R> u[W];
       project_row<R, W>(Ub + (size_t)q * nb + i, u);
-      const cplx<R>* fr = f + ((size_t)bf[xb] * nrhs + r0) * Ef + e;
+      const cplx<R>* fr = f + (size_t)bf[xb] * nr * Ef + e;
 #pragma unroll
       for (int r = 0; r < RCT; ++r)
         if (r < nr) {
@@ -240,30 +226,29 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
         for (int k = 0; k < 2; ++k)
 #pragma unroll
           for (int w = 0; w < W; ++w)
-            s_red[(((size_t)g * RC + r) * 2 + k) * nb + i + w] = acc[r][k][w];
+            s_red[(((size_t)g * RCT + r) * 2 + k) * nb + i + w] = acc[r][k][w];
   }
   __syncthreads();
-  for (int o = tid; o < nr * 2 * nb; o += blockDim.x) {
-    const int r = o / (2 * nb), kn = o - r * 2 * nb;  // kn = k*nb + i
+  for (int o = tid; o < nr * 2 * nb; o += blockDim.x) {  // o = (r*2 + k)*nb + i
     cplx<R> t = {R(0), R(0)};
-    for (int gg = 0; gg < G; ++gg) t = cadd(t, s_red[((size_t)gg * RC + r) * 2 * nb + kn]);
+    for (int gg = 0; gg < G; ++gg) t = cadd(t, s_red[(size_t)gg * RCT * 2 * nb + o]);
     if (gridDim.z == 1)
-      c[((size_t)xc * nrhs + r0 + r) * 2 * nb + kn] = t;
+      c[(size_t)xc * nr * 2 * nb + o] = t;
     else
-      part[(((size_t)xc * gridDim.y + blockIdx.y) * gridDim.z + blockIdx.z) * RC * 2 * nb + o] = t;
+      part[((size_t)xc * gridDim.z + blockIdx.z) * nr * 2 * nb + o] = t;
   }
 }
 
-// c(xc)(y*RC + r)(kn) = sum over the S row ranges of the partial sums.  One
-// workgroup per (xc, y): thread (o, zg) sums z = zg, zg + ZG, ... for output
+// c(xc)(y*rc + r)(kn) = sum over the S row ranges of the partial sums, rp =
+// min(rc, nrhs) rhs a row of them.  One workgroup per (xc, y): thread (o, zg) sums z = zg, zg + ZG, ... for output
 // o, and the ZG group sums are added in order in LDS.
 template <typename R>
 __global__ __launch_bounds__(256) void k_project_reduce(const cplx<R>* __restrict__ part,
                                                         cplx<R>* __restrict__ c, int nchunk,
-                                                        int S, int nrhs, int nb) {
+                                                        int S, int nrhs, int nb, int rc, int rp) {
   extern __shared__ unsigned char smem_raw[];
-  cplx<R>* s_acc = reinterpret_cast<cplx<R>*>(smem_raw);  // [ZG][RC*2*nb]
-  const int no = RC * 2 * nb;
+  cplx<R>* s_acc = reinterpret_cast<cplx<R>*>(smem_raw);  // [ZG][rp*2*nb]
+  const int no = rp * 2 * nb;
   const size_t xy = blockIdx.x;
   const int y = (int)(xy % nchunk), xc = (int)(xy / nchunk);
   if (no > (int)blockDim.x) {  // wide outputs: one thread per output, z in order
@@ -271,7 +256,7 @@ __global__ __launch_bounds__(256) void k_project_reduce(const cplx<R>* __restric
       cplx<R> t = {R(0), R(0)};
       for (int z = 0; z < S; ++z) t = cadd(t, part[(xy * S + z) * no + oo]);
       const int r = oo / (2 * nb), kn = oo - r * 2 * nb;
-      if (y * RC + r < nrhs) c[((size_t)xc * nrhs + y * RC + r) * 2 * nb + kn] = t;
+      if (y * rc + r < nrhs) c[((size_t)xc * nrhs + y * rc + r) * 2 * nb + kn] = t;
     }
     return;
   }
@@ -286,38 +271,50 @@ __global__ __launch_bounds__(256) void k_project_reduce(const cplx<R>* __restric
     cplx<R> t = {R(0), R(0)};
     for (int g = 0; g < ZG; ++g) t = cadd(t, s_acc[g * no + oo]);
     const int r = oo / (2 * nb), kn = oo - r * 2 * nb;
-    if (y * RC + r < nrhs) c[((size_t)xc * nrhs + y * RC + r) * 2 * nb + kn] = t;
+    if (y * rc + r < nrhs) c[((size_t)xc * nrhs + y * rc + r) * 2 * nb + kn] = t;
   }
 }
 
+template <typename R>
+void project_reduce(const cplx<R>* part, cplx<R>* out, int Vc, int nchunk, int S, int nrhs, int nb,
+                    int rc, hipStream_t s) {
+  // ZG * (rp*2*nb) <= 256 entries of LDS
+  k_project_reduce<R><<<Vc * nchunk, 256, 256 * sizeof(cplx<R>), s>>>(
+      part, out, nchunk, S, nrhs, nb, rc, std::min(rc, nrhs));
+  MGC_LAUNCH_CHECK();
+}
+
+template void project_reduce<float>(const cplx<float>*, cplx<float>*, int, int, int, int, int, int,
+                                    hipStream_t);
+template void project_reduce<double>(const cplx<double>*, cplx<double>*, int, int, int, int, int,
+                                     int, hipStream_t);
+
 // ---------------------------------------------------------------------------
 // promote: f(fine(xc,xb))(rhs)(e) = sum_i c(xc)(rhs)(chirality(e), i) U(xc,xb,e,i)
-// One workgroup per (coarse site, chunk of RC right-hand sides).  The block's
-// basis panel (rows q = (xb, e), nb entries each, row-major) is streamed in
+// for one rhs (RCT = 1) or up to four (RCT = 4; wider calls: transfer_mfma.hip).
+// One workgroup per coarse site.  The block's basis panel (rows q = (xb, e), nb entries each, row-major) is streamed in
 // tiles of 256/LPR rows: each tile is read with contiguous loads
 // (consecutive threads take consecutive panel entries), stored transposed in
 // LDS ([i][row], one row of padding against bank conflicts), and each group of
 // LPR adjacent lanes then sums one row, nb/LPR entries each, joined by lane
 // exchanges.  LPR = 2, or 4 where a 128-row tile would not fit in 64 KB.
 // ---------------------------------------------------------------------------
-template <typename R, int LPR, int TPT>
+template <typename R, int RCT, int LPR, int TPT>
 __global__ __launch_bounds__(256) void k_promote(const cplx<R>* __restrict__ U,
                                                  const cplx<R>* __restrict__ c,
                                                  cplx<R>* __restrict__ f,
                                                  const int* __restrict__ blk_fine, int nb, int Vb,
-                                                 int Ef, int nrhs, int rows_per) {
+                                                 int Ef, int nr, int rows_per) {
   extern __shared__ unsigned char smem_raw[];
-  cplx<R>* s_c = reinterpret_cast<cplx<R>*>(smem_raw);  // [RC][2][nb]
+  cplx<R>* s_c = reinterpret_cast<cplx<R>*>(smem_raw);  // [RCT][2][nb]
   constexpr int PR = 256 / LPR;                         // rows per tile
   constexpr int LD = PR + 1;
-  cplx<R>* s_u = s_c + RC * 2 * nb;                     // [nb][LD]
+  cplx<R>* s_u = s_c + RCT * 2 * nb;                    // [nb][LD]
   const int xc = blockIdx.x;
-  const int r0 = blockIdx.y * RC;
-  const int nr = min(RC, nrhs - r0);
   const int tid = threadIdx.x;
   const int half = Ef / 2;
   for (int o = tid; o < nr * 2 * nb; o += blockDim.x)
-    s_c[o] = c[((size_t)xc * nrhs + r0) * 2 * nb + o];
+    s_c[o] = c[(size_t)xc * nr * 2 * nb + o];
   const int rows = Vb * Ef;
   const cplx<R>* Ub = U + (size_t)xc * rows * nb;
   const int* bf = blk_fine + (size_t)xc * Vb;
@@ -367,25 +364,23 @@ __global__ __launch_bounds__(256) void k_promote(const cplx<R>* __restrict__ U,
     // the next tile (after the last one, the current tile again: L2 hits,
     // never stored; keeps the prefetch unconditional)
     fetch(q0 + PR < qend ? q0 + PR : q0);
-    cplx<R> acc[RC];
+    cplx<R> acc[RCT];
 #pragma unroll
-    for (int r = 0; r < RC; ++r) acc[r] = {R(0), R(0)};
+    for (int r = 0; r < RCT; ++r) acc[r] = {R(0), R(0)};
     const bool active = row_l < nrow;
-    int k = 0;
     if (active) {
-      const int q = q0 + row_l;
-      k = (q % Ef) >= half;
+      const int k = (q0 + row_l) % Ef >= half;
       for (int i = i0; i < i1; ++i) {
         const cplx<R> u = s_u[i * LD + row_l];
 #pragma unroll
-        for (int r = 0; r < RC; ++r)
+        for (int r = 0; r < RCT; ++r)
           if (r < nr) cmac(acc[r], s_c[(r * 2 + k) * nb + i], u);
       }
     }
 #pragma unroll
     for (int off = 1; off < LPR; off <<= 1)
 #pragma unroll
-      for (int r = 0; r < RC; ++r) {
+      for (int r = 0; r < RCT; ++r) {
         acc[r].re += __shfl_xor(acc[r].re, off);
         acc[r].im += __shfl_xor(acc[r].im, off);
       }
@@ -393,8 +388,8 @@ __global__ __launch_bounds__(256) void k_promote(const cplx<R>* __restrict__ U,
       const int q = q0 + row_l;
       const int xb = q / Ef, e = q - xb * Ef;
 #pragma unroll
-      for (int r = 0; r < RC; ++r)
-        if (r < nr) f[((size_t)bf[xb] * nrhs + r0 + r) * Ef + e] = acc[r];
+      for (int r = 0; r < RCT; ++r)
+        if (r < nr) f[((size_t)bf[xb] * nr + r) * Ef + e] = acc[r];
     }
   }
 }
@@ -896,33 +891,47 @@ static void check_agg(const mgc_aggregation* a) {
   MGC_CHECK(a->basis_set, MGC_ERR_STATE, "basis not set");
 }
 
+// FP64 promote takes at most 56 basis vectors, for one rhs (64 KB of LDS with
+// the four-lane tile) and for several alike
+static bool promote_nb_ok(int prec, int nb) { return prec != MGC_F64 || nb <= 56; }
+static const char* const PROMOTE_NB_MSG = "promote: nbasis too large for the LDS tile";
+
 void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int nrhs,
                   bool project, int kind, int point, hipStream_t s) {
   check_agg(a);
   MGC_CHECK(in && out && in != out, MGC_ERR_ARG, "null or aliased vector");
   MGC_CHECK(nrhs >= 1, MGC_ERR_ARG, "nrhs < 1");
-  const int nchunk = (nrhs + RC - 1) / RC;
+  MGC_CHECK(prec == MGC_F64 || prec == MGC_F32, MGC_ERR_PRECISION,
+            project ? "project: F64 or F32 vectors" : "promote: F64 or F32 vectors");
   const int nb = a->nb;
   const int rows = a->Vb * a->Ef;
+  // The matrix form reads the basis once per 16 rhs, the vector forms once per
+  // four, but its 16 x 16 tiles are mostly padding when both nb and nrhs are
+  // small.  Matrix over vector time at (nb, nrhs), project + promote over 16^3 x
+  // 32 and 18^4 with 3^4 blocks: (12, 2), (12, 3) 1.06 to 1.3, (20, 3) 0.91 to
+  // 1.24, (16, 4), (24, 3), (32, 2) 0.73 to 1.04, more than four rhs at most
+  // 0.83; in FP64, where the products weigh more, (20, 4) 0.98 to 1.18.
+  const bool full_tiles = prec == MGC_F32 || 4 * nb >= 3 * ((nb + 15) / 16 * 16);
+  const bool matrix = nrhs > 4 || (nrhs * nb >= 64 && full_tiles);
+  const int rct = nrhs == 1 ? 1 : 4;
   // split each panel over S workgroups when the coarse lattice alone gives
-  // fewer than ~1024 workgroups (at least 64 rows per workgroup)
+  // fewer than ~1024 workgroups (at least 64 rows per workgroup; a workgroup
+  // of four rhs counted, the split of several rhs needs no more than that)
+  const size_t wgs = (size_t)a->Vc * ((nrhs + 3) / 4);
   int S = 1;
-  if ((size_t)a->Vc * nchunk < 1024) {
-    S = (int)((1024 + (size_t)a->Vc * nchunk - 1) / ((size_t)a->Vc * nchunk));
+  if (wgs < 1024) {
+    S = (int)((1024 + wgs - 1) / wgs);
     S = std::min(S, std::max(1, rows / 64));
   }
   const int rows_per = (rows + S - 1) / S;
   S = (rows + rows_per - 1) / rows_per;
-  const dim3 grid(a->Vc, nchunk, S);
+  const dim3 grid(a->Vc, 1, S);
   const size_t es = prec == MGC_F64 ? sizeof(cplx<double>) : sizeof(cplx<float>);
   if (project) {
-    MGC_CHECK(prec == MGC_F64 || prec == MGC_F32, MGC_ERR_PRECISION,
-              "project: F64 or F32 vectors");
-    const int block = (256 / nb) * nb;
-    const size_t sh = (size_t)(block / nb) * RC * 2 * nb * es;
     void* part = nullptr;
     if (S > 1) {
-      const size_t need = (size_t)a->Vc * nchunk * S * RC * 2 * nb * es;
+      const size_t need =
+          (size_t)a->Vc * ((nrhs + 15) / 16) * S * std::min(16, nrhs) * 2 * nb * es;
       if (need > a->part_bytes) {
         if (a->part) MGC_HIP(hipFree(a->part));
         a->part = nullptr;
@@ -932,69 +941,66 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
       }
       part = a->part;
     }
-    const int nred = a->Vc * nchunk;  // reduction workgroups
-    const size_t red_sh = (size_t)256 * es;  // ZG * (RC*2*nb) <= 256 entries
+    // even nb in FP32: two adjacent columns per thread in one 16-byte load
+    const int w = prec == MGC_F32 && nb % 2 == 0 ? 2 : 1;
+    const int G = 256 / (nb / w), block = G * (nb / w);
+    const size_t sh = (size_t)G * rct * 2 * nb * es;
+#define PROJECT_T(R, RCT, W, basis)                                                           \
+  k_project<R, RCT, W><<<grid, block, sh, s>>>(basis, (const cplx<R>*)in, (cplx<R>*)out,      \
+                                               a->blk_fine, nb, a->Vb, a->Ef, nrhs, a->blk,   \
+                                               kind, point, rows_per, (cplx<R>*)part)
+#define PROJECT(R, W, basis)                                                                  \
+  do {                                                                                        \
+    if (rct == 1) PROJECT_T(R, 1, W, basis);                                                  \
+    else PROJECT_T(R, 4, W, basis);                                                           \
+    if (S > 1)                                                                                \
+      project_reduce<R>((const cplx<R>*)part, (cplx<R>*)out, a->Vc, 1, S, nrhs, nb, 4, s);    \
+  } while (0)
     if (prec == MGC_F64) {
-      if (nrhs == 1)
-        k_project<double, 1><<<grid, block, sh, s>>>(a->basis64, (const cplx<double>*)in,
-                                                     (cplx<double>*)out, a->blk_fine, nb, a->Vb,
-                                                     a->Ef, nrhs, a->blk, kind, point, rows_per,
-                                                     (cplx<double>*)part);
+      if (matrix)
+        project_mfma<double>(a, a->basis64, (const cplx<double>*)in, (cplx<double>*)out,
+                             (cplx<double>*)part, nrhs, S, kind, point, s);
       else
-        k_project<double, RC><<<grid, block, sh, s>>>(a->basis64, (const cplx<double>*)in,
-                                                      (cplx<double>*)out, a->blk_fine, nb, a->Vb,
-                                                      a->Ef, nrhs, a->blk, kind, point, rows_per,
-                                                      (cplx<double>*)part);
-      if (S > 1)
-        k_project_reduce<double><<<nred, 256, red_sh, s>>>((const cplx<double>*)part,
-                                                            (cplx<double>*)out, nchunk, S, nrhs,
-                                                            nb);
+        PROJECT(double, 1, a->basis64);
     } else {
       const cplx<float>* b32 = agg_basis32(a, s);
-      // even nb: two adjacent columns per thread in one 16-byte load
-      const bool paired = nb % 2 == 0;
-      const int block2 = (256 / (nb / 2 > 0 ? nb / 2 : 1)) * (nb / 2);
-      const size_t sh2 = (size_t)(paired ? block2 / (nb / 2) : 0) * RC * 2 * nb * es;
-      if (paired && nrhs == 1)
-        k_project<float, 1, 2><<<grid, block2, sh2, s>>>(b32, (const cplx<float>*)in,
-                                                         (cplx<float>*)out, a->blk_fine, nb,
-                                                         a->Vb, a->Ef, nrhs, a->blk, kind, point,
-                                                         rows_per, (cplx<float>*)part);
-      else if (paired)
-        k_project<float, RC, 2><<<grid, block2, sh2, s>>>(b32, (const cplx<float>*)in,
-                                                          (cplx<float>*)out, a->blk_fine, nb,
-                                                          a->Vb, a->Ef, nrhs, a->blk, kind, point,
-                                                          rows_per, (cplx<float>*)part);
-      else if (nrhs == 1)
-        k_project<float, 1><<<grid, block, sh, s>>>(b32, (const cplx<float>*)in,
-                                                    (cplx<float>*)out, a->blk_fine, nb, a->Vb,
-                                                    a->Ef, nrhs, a->blk, kind, point, rows_per,
-                                                    (cplx<float>*)part);
+      if (matrix)
+        project_mfma<float>(a, b32, (const cplx<float>*)in, (cplx<float>*)out,
+                            (cplx<float>*)part, nrhs, S, kind, point, s);
+      else if (w == 2)
+        PROJECT(float, 2, b32);
       else
-        k_project<float, RC><<<grid, block, sh, s>>>(b32, (const cplx<float>*)in,
-                                                     (cplx<float>*)out, a->blk_fine, nb, a->Vb,
-                                                     a->Ef, nrhs, a->blk, kind, point, rows_per,
-                                                     (cplx<float>*)part);
-      if (S > 1)
-        k_project_reduce<float><<<nred, 256, red_sh, s>>>((const cplx<float>*)part,
-                                                           (cplx<float>*)out, nchunk, S, nrhs,
-                                                           nb);
+        PROJECT(float, 1, b32);
     }
+#undef PROJECT
+#undef PROJECT_T
+  } else if (matrix) {
+    MGC_CHECK(promote_nb_ok(prec, nb), MGC_ERR_SHAPE, PROMOTE_NB_MSG);
+    if (prec == MGC_F64)
+      promote_mfma<double>(a, a->basis64, (const cplx<double>*)in, (cplx<double>*)out, nrhs, s);
+    else
+      promote_mfma<float>(a, agg_basis32(a, s), (const cplx<float>*)in, (cplx<float>*)out, nrhs,
+                          s);
   } else {
-    auto lds = [&](int lpr) { return ((size_t)RC * 2 * nb + (size_t)nb * (256 / lpr + 1)) * es; };
+    MGC_CHECK(promote_nb_ok(prec, nb), MGC_ERR_SHAPE, PROMOTE_NB_MSG);
+    auto lds = [&](int lpr) {
+      return ((size_t)rct * 2 * nb + (size_t)nb * (256 / lpr + 1)) * es;
+    };
     // FP32 with nb <= 32: one lane per row, 256-row tiles (half the barriers
     // per panel); otherwise two (or four) lanes per row
     const int lpr = prec == MGC_F32 && nb <= 32 && lds(1) <= 65536 ? 1
                     : lds(2) <= 65536                               ? 2
                                                                     : 4;
     const size_t sh = lds(lpr);
-    MGC_CHECK(sh <= 65536, MGC_ERR_SHAPE, "promote: nbasis too large for the LDS tile");
     // register prefetch depth: entries per thread of one tile, rounded up to a power of 2
     const int need = (256 / lpr * nb + 255) / 256;
     const int tpt = need <= 2 ? 2 : need <= 4 ? 4 : need <= 8 ? 8 : need <= 16 ? 16 : 32;
-#define PROMOTE_T(R, LPR, T, basis)                                                            \
-  k_promote<R, LPR, T><<<grid, 256, sh, s>>>(basis, (const cplx<R>*)in, (cplx<R>*)out,          \
-                                             a->blk_fine, nb, a->Vb, a->Ef, nrhs, rows_per)
+#define PROMOTE_R(R, RCT, LPR, T, basis)                                                      \
+  k_promote<R, RCT, LPR, T><<<grid, 256, sh, s>>>(basis, (const cplx<R>*)in, (cplx<R>*)out,   \
+                                                  a->blk_fine, nb, a->Vb, a->Ef, nrhs, rows_per)
+#define PROMOTE_T(R, LPR, T, basis)          \
+  if (rct == 1) PROMOTE_R(R, 1, LPR, T, basis); \
+  else PROMOTE_R(R, 4, LPR, T, basis)
 #define PROMOTE(R, LPR, basis)                           \
   switch (tpt) {                                         \
     case 2: PROMOTE_T(R, LPR, 2, basis); break;          \
@@ -1009,7 +1015,7 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
       } else {
         PROMOTE(double, 4, a->basis64)
       }
-    } else if (prec == MGC_F32) {
+    } else {
       if (lpr == 1) {
         PROMOTE(float, 1, agg_basis32(a, s))
       } else if (lpr == 2) {
@@ -1017,11 +1023,10 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
       } else {
         PROMOTE(float, 4, agg_basis32(a, s))
       }
-    } else {
-      throw Error(MGC_ERR_PRECISION, "promote: F64 or F32 vectors");
     }
 #undef PROMOTE
 #undef PROMOTE_T
+#undef PROMOTE_R
   }
   MGC_LAUNCH_CHECK();
 }

@@ -34,11 +34,35 @@ const cplx<float>* agg_basis32(mgc_aggregation* a, hipStream_t s);
 // project (mask kind 0 all / 1 inner of point / 2 outer of point) or promote
 void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int nrhs,
                   bool project, int kind, int point, hipStream_t s);
+// project / promote of several right-hand sides on the matrix cores
+// (transfer_mfma.hip).  S row ranges per block; part: workspace of
+// Vc * ceil(nrhs / 16) * S * min(16, nrhs) * 2 nb entries where S > 1
+template <typename R>
+void project_mfma(const mgc_aggregation* a, const cplx<R>* U, const cplx<R>* in, cplx<R>* out,
+                  cplx<R>* part, int nrhs, int S, int kind, int point, hipStream_t s);
+template <typename R>
+void promote_mfma(const mgc_aggregation* a, const cplx<R>* U, const cplx<R>* in, cplx<R>* out,
+                  int nrhs, hipStream_t s);
+// out = the sums over the S ranges of part ([Vc][nchunk][S][min(rc, nrhs)][2 nb])
+template <typename R>
+void project_reduce(const cplx<R>* part, cplx<R>* out, int Vc, int nchunk, int S, int nrhs, int nb,
+                    int rc, hipStream_t s);
 // fine field [Vf][Ef] holding the chirality-l part of basis vector i (l = -1: all)
 void agg_extract_basis(mgc_aggregation* a, int i, int l, void* out, int prec, hipStream_t s);
 // FP64 fine fields [Vf][nr][Ef] of the doubled basis columns n0 .. n0+nr-1
 // (column n = chirality-(n / nb) part of basis vector n % nb)
 void agg_extract_doubled(mgc_aggregation* a, int n0, int nr, void* out, hipStream_t s);
+// Site mask of a block site: kind 0 = all, 1 = inner of point p, 2 = outer of
+// point p (outer for +mu: x_mu mod b = b-1; for -mu: x_mu mod b = 0).
+__device__ inline bool site_in_mask(const Lat4& blk, int xb, int kind, int p) {
+  if (kind == 0 || p == 8) return kind != 2;
+  int c[4];
+  blk.coords(xb, c);
+  const int mu = p & 3;
+  const bool outer = c[mu] == (p < 4 ? blk.L[mu] - 1 : 0);
+  return kind == 2 ? outer : !outer;
+}
+
 __host__ __device__ inline size_t agg_row(int nb, int Vb, int Ef, int xc, int xb, int e) {
   return (((size_t)xc * Vb + xb) * Ef + e) * nb;
 }

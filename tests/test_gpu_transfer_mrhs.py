@@ -1,0 +1,101 @@
+"""Project and promote of several right-hand sides (the matrix-core form) at the
+edges of its tiles: basis widths around multiples of 16 and 4 (odd ones among
+them), 16-rhs column tiles with remainders, blocks whose site count is no
+multiple of a wavefront's four or sixteen sites, fields of a coarse level
+(element counts other than 12), masks, panels split over workgroups, and FP32
+fields at an address that is no multiple of 16 bytes.
+
+Tolerances as in test_gpu_aggregation.py: relative L2 1e-13 in FP64 and 2e-6 in
+FP32, where basis and inputs are rounded to 2^-24 and the sums are FP32.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import gauss, rel
+
+pytestmark = pytest.mark.gpu
+
+# fine lattice, block, nb, elements per site, nrhs
+SHAPES = [
+    ((4, 4, 4, 4), (4, 4, 4, 4), 16, 12, 12),   # one block, split over workgroups
+    ((4, 4, 2, 4), (2, 2, 1, 2), 1, 12, 2),
+    ((4, 2, 2, 4), (2, 2, 2, 2), 7, 12, 16),
+    ((3, 3, 6, 3), (3, 3, 3, 3), 12, 12, 17),   # 81 sites a block, two column tiles
+    ((6, 3, 3, 3), (3, 3, 3, 3), 20, 12, 3),
+    ((8, 4, 4, 4), (4, 4, 4, 2), 24, 12, 5),
+    ((4, 4, 4, 4), (2, 2, 2, 2), 17, 12, 33),
+    ((4, 4, 4, 4), (4, 2, 2, 1), 33, 12, 4),
+    ((4, 4, 2, 2), (2, 2, 2, 2), 48, 12, 12),
+    ((4, 4, 4, 4), (2, 2, 2, 2), 56, 12, 7),
+    ((4, 4, 4, 4), (2, 2, 2, 2), 16, 32, 12),   # a coarse level's field
+    ((2, 2, 4, 2), (2, 2, 2, 2), 6, 6, 2),      # three elements per chirality
+    ((2, 4, 2, 2), (2, 1, 2, 2), 10, 26, 19),
+    ((16, 16, 8, 8), (2, 2, 2, 2), 8, 12, 2),   # 1024 blocks, no split
+    ((6, 3, 3, 3), (3, 3, 3, 3), 5, 12, 8),     # at most 8 columns and 8 rhs, 81 sites
+    ((4, 4, 4, 4), (2, 2, 4, 4), 8, 12, 9),
+]
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("fd,blk,nb,Ef,nrhs", SHAPES)
+def test_transfers_match_oracle(gpu, fd, blk, nb, Ef, nrhs, prec):
+    print(f"[case] fd={fd} blk={blk} nb={nb} Ef={Ef} nrhs={nrhs} prec={prec}", flush=True)
+    Vf, Vc = int(np.prod(fd)), int(np.prod(oracle.coarse_dims(fd, blk)))
+    dt = gpu.complex_dtype(prec)
+    sz = np.dtype(dt).itemsize
+    tol = 1e-13 if prec == 0 else 2e-6
+    B = gauss(nb * Vf * Ef, 801).reshape(nb, Vf, Ef)
+    agg = gpu.Aggregation(fd, blk, nb, Ef)
+    agg.set_basis(gpu.DeviceBuffer.from_numpy(B))
+    f = gauss(Vf * nrhs * Ef, 802).reshape(Vf, nrhs, Ef).astype(dt)
+    c = gauss(Vc * nrhs * 2 * nb, 803).reshape(Vc, nrhs, 2 * nb).astype(dt)
+    ref_c, ref_f = [], []
+    for r in range(nrhs):
+        ref_c.append(oracle.project_ef(fd, blk, nb, Ef, B, f[:, r].astype(np.complex128)))
+        ref_f.append(oracle.promote_ef(fd, blk, nb, Ef, B, c[:, r].astype(np.complex128)))
+    ref_c, ref_f = np.stack(ref_c, 1), np.stack(ref_f, 1)
+    for shift in (0, 1):  # the fields one complex number into their buffers
+        pad = np.zeros(shift, dt)
+        df = gpu.DeviceBuffer.from_numpy(np.concatenate([pad, f.ravel()]))
+        dc = gpu.DeviceBuffer.from_numpy(np.concatenate([pad, c.ravel()]))
+        oc = gpu.DeviceBuffer(Vc * nrhs * 2 * nb * sz)
+        of = gpu.DeviceBuffer((f.size + 2 * shift) * sz)
+        of.zero()
+        agg.project(df.ptr + shift * sz, oc, prec, nrhs)
+        agg.promote(dc.ptr + shift * sz, of.ptr + shift * sz, prec, nrhs)
+        gpu.synchronize()
+        got_c = oc.to_numpy(dt, ref_c.shape)
+        raw = of.to_numpy(dt, (f.size + 2 * shift,))
+        got_f = raw[shift:shift + f.size].reshape(ref_f.shape)
+        for r in range(nrhs):
+            assert rel(ref_c[:, r], got_c[:, r].astype(np.complex128)) < tol, (shift, r)
+            assert rel(ref_f[:, r], got_f[:, r].astype(np.complex128)) < tol, (shift, r)
+        assert not raw[:shift].any() and not raw[shift + f.size:].any()
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+def test_masked_project_of_many_rhs(gpu, prec):
+    """Inner and outer sites of each point on blocks with an odd extent."""
+    fd, blk, nb, nrhs = (6, 4, 4, 3), (3, 2, 4, 3), 18, 18
+    print(f"[case] masked fd={fd} blk={blk} nb={nb} nrhs={nrhs} prec={prec}", flush=True)
+    Vf, Vc = int(np.prod(fd)), int(np.prod(oracle.coarse_dims(fd, blk)))
+    dt = gpu.complex_dtype(prec)
+    tol = 1e-13 if prec == 0 else 2e-6
+    B = gauss(nb * Vf * 12, 811).reshape(nb, Vf, 12)
+    agg = gpu.Aggregation(fd, blk, nb)
+    agg.set_basis(gpu.DeviceBuffer.from_numpy(B))
+    f = gauss(Vf * nrhs * 12, 812).reshape(Vf, nrhs, 12).astype(dt)
+    df = gpu.DeviceBuffer.from_numpy(f)
+    dc = gpu.DeviceBuffer(Vc * nrhs * 2 * nb * np.dtype(dt).itemsize)
+    for point in range(9):
+        for kind in (0, 1, 2):
+            if kind == 2 and point == 8:
+                continue  # no site is outside the self point
+            agg.project_masked(df, dc, kind, point, prec, nrhs)
+            gpu.synchronize()
+            got = dc.to_numpy(dt, (Vc, nrhs, 2 * nb)).astype(np.complex128)
+            for r in (0, 7, nrhs - 1):
+                ref = oracle.project(fd, blk, nb, B, f[:, r].astype(np.complex128), kind=kind,
+                                     point=point)
+                assert rel(ref, got[:, r]) < tol, (point, kind, r)
