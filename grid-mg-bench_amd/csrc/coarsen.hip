@@ -324,42 +324,134 @@ __global__ __launch_bounds__(4 * (NB / TC) * (NB / TC)) void k_coarsen(
 // so that C'[c][2c'+v] = (Re, Im) C[c][c'].  Rows and columns past NB are zero
 // padding of the 16 x 16 tiles and are never stored.  The staged u and W are
 // kept as separate real and imaginary planes in LDS, so every lane's operand
-// is one 8-byte read.  W is built on the vector ALU as in the FP64 form.
+// is one 8-byte read.
 // MFMA 16x16x4 f64 lane layout: A[i = l%16][k = l/16], B[k = l/16][j = l%16],
 // D[i = 4r + l/16][j = l%16] for result r < 4 (rows interleaved, unlike the
 // FP32 16x16x4 form's 4(l/16) + r).
-constexpr int CM_SB = 4;  // fine sites per stage
+//
+// What bounds it: the products (412 GFLOP at 32^4, 4^4 blocks, nb 32: 5.7 ms at
+// the FP64 matrix rate) and, for the self point, the gathers of W: the panel
+// comes from beyond L2 three times (20 GB).  The workgroups of a CU overlap the
+// two, so a stage is sized for three of them (38 KB of LDS: two sites at nb >
+// 16, four below; up to 168 registers a lane).  For the registers a W item is
+// one spin of one chirality (two lanes per column), the link, the same for a
+// whole wavefront, is read into scalar registers, and the faces and the self
+// point are kernels of their own.  Faces 4.7 ms (62% of the matrix rate), self
+// 9.3 ms; one kernel at two workgroups a CU and a lane per column: 18.2 ms.
+// All of a stage's loads in flight one stage ahead, at two workgroups: 16.5 ms.
+constexpr int co_sites(int nb) { return nb > 16 ? 2 : 4; }  // fine sites per stage
 typedef double doublex4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) double* scalar_f64_ptr;
 
-template <int NB>
-__global__ __launch_bounds__(256) void k_coarsen_mfma(
+// the value of the neighbouring lane l ^ 1
+__device__ __forceinline__ double swap_pair(double x) {
+  union { double d; int i[2]; } a, b;
+  a.d = x;
+#pragma unroll
+  for (int k = 0; k < 2; ++k)  // quad permutation (1, 0, 3, 2)
+    b.i[k] = __builtin_amdgcn_mov_dpp(a.i[k], 0xB1, 0xF, 0xF, true);
+  return b.d;
+}
+
+// One hop of one W item: lane (cp, sl) of chirality lw adds its spin's part of
+// H_q P_lw u_cp to ws (spin 2 lw + sl) and the gamma image to wo (the spin of
+// the other chirality that g_mu maps it to).  U: the link, B: the lane's three
+// colours of the neighbour; bit mu of neg: the image spin's phase is negative.
+template <int Q>
+__device__ __forceinline__ void coarsen_hop(unsigned neg, scalar_f64_ptr U,
+                                            const cplx<double> B[3], cplx<double> ws[3],
+                                            cplx<double> wo[3]) {
+  constexpr int mu = Q & 3;
+  // half the phase of the image spin, +-1 (y, t) or +-i (x, z): bit mu of neg
+  const double f =
+      __hiloint2double((int)(0x3fe00000u ^ (((neg >> mu) ^ (Q < 4 ? 0u : 1u)) << 31)), 0);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    cplx<double> chi = {0.0, 0.0};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      // row i of U (forward) or of U^dag (backward)
+      const int k = Q < 4 ? i * 3 + j : j * 3 + i;
+      const cplx<double> l = {U[2 * k], Q < 4 ? U[2 * k + 1] : -U[2 * k + 1]};
+      cmac(chi, l, B[j]);
+    }
+    ws[i].re -= 0.5 * chi.re;
+    ws[i].im -= 0.5 * chi.im;
+    if (mu % 2) {
+      wo[i].re += f * chi.re;
+      wo[i].im += f * chi.im;
+    } else {
+      wo[i].re -= f * chi.im;
+      wo[i].im += f * chi.re;
+    }
+  }
+}
+
+template <int NB, bool SELF>
+__global__ __launch_bounds__(256, 3) void k_coarsen_mfma(
     const cplx<double>* __restrict__ basis, const cplx<double>* __restrict__ gauge,
     const cplx<double>* __restrict__ diag, Lat4 fine, Lat4 coarse, Lat4 blk, int Vf, int Vb,
     const int* __restrict__ plist, int np, int Vc, cplx<double>* __restrict__ links) {
+  constexpr int SB = co_sites(NB);
   constexpr int MT = (NB + 15) / 16;   // m-tiles (rows c)
   constexpr int NTL = (NB + 7) / 8;    // n-tiles (columns 2c'+v)
   constexpr int NBP = NB + 1;          // LDS row pitch (doubles) against bank conflicts
   constexpr int ROW = 12 * NB;
-  static_assert(CM_SB == 4 && NB <= 32, "one stage site per wavefront, 2 NB lanes per site");
-  __shared__ double sUr[CM_SB][12][NBP], sUi[CM_SB][12][NBP];      // u, with -Im u
-  __shared__ double sWr[CM_SB][2][12][NBP], sWi[CM_SB][2][12][NBP];  // W
-  const GammaTab G = gamma_table();
+  constexpr int LPS = 256 / SB;        // lanes that build one site
+  constexpr int NU = (ROW + LPS - 1) / LPS;  // staged u entries per lane
+  constexpr int PL = SB * 12 * NBP;    // one plane of u; a plane of W is two
+  static_assert(NB <= 32, "lanes of a W item");
+  __shared__ double smem[6 * PL];
+  double* const sUr = smem;            // u[site][e][c], with -Im u in sUi
+  double* const sUi = smem + PL;
+  double* const sWr = smem + 2 * PL;   // W[site][l][e][c']
+  double* const sWi = smem + 4 * PL;
 
   int xc, pi;
   coarsen_work((int)blockIdx.x, np, Vc, xc, pi);
-  const CoGeom g(basis, gauge, diag, fine, coarse, blk, Vf, Vb, xc, plist[pi]);
+  // the same for all lanes, though divisions computed them in vector registers
+  xc = __builtin_amdgcn_readfirstlane(xc);
+  pi = __builtin_amdgcn_readfirstlane(pi);
+  CoGeom g(basis, gauge, diag, fine, coarse, blk, Vf, Vb, xc, SELF ? 8 : plist[pi]);
+#pragma unroll
+  for (int d = 0; d < 4; ++d) g.cc[d] = __builtin_amdgcn_readfirstlane(g.cc[d]);
+  g.nsite = __builtin_amdgcn_readfirstlane(g.nsite);
+  const int p = SELF ? 8 : g.p;
   const int tid = threadIdx.x;
-  const int w = tid >> 6, l = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63;
   const int kb = w >> 1, lb = w & 1;  // chirality block of this wavefront
   const int lk = l >> 4;              // k index of this lane within a k-step
   const int t = lk & 1;               // real (0) or imaginary (1) slot of K
   // A operand: row c = mt*16 + l%16, from the plane of t
-  const double* aplane = t ? &sUi[0][0][0] : &sUr[0][0][0];
+  const double* aplane = t ? sUi : sUr;
   // B operand: column n = nt*16 + l%16, c' = n/2, v = n%2: plane Re for
   // t == v, else Im, negated for (t, v) = (1, 0)
   const int v = l & 1;
-  const double* bplane = (t ^ v) ? &sWi[0][0][0][0] : &sWr[0][0][0][0];
+  const double* bplane = (t ^ v) ? sWi : sWr;
   const double bsign = (t == 1 && v == 0) ? -1.0 : 1.0;
+
+  // W item of this lane: site ss of the stage (uniform over the wavefront),
+  // chirality lw, spin 2 lw + sl, column cp
+  const int ss = SB == 2 ? w >> 1 : w;
+  const int lw = SB == 2 ? w & 1 : l >> 5;
+  const int sl = l & 1;
+  const int cp_raw = (SB == 2 ? l : l & 31) >> 1;
+  const bool col = cp_raw < NB;
+  const int cp = col ? cp_raw : NB - 1;
+  const int e0 = 6 * lw + 3 * sl;  // first of this lane's elements
+  const int li = SB == 2 ? tid & 127 : l;  // lane among those of the site
+
+  unsigned neg = 0;  // bit mu: sign of the phase of this lane's image spin under g_mu
+  {
+    const GammaTab G = gamma_table();
+#pragma unroll
+    for (int mu = 0; mu < 4; ++mu)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const int s2 = G.col[mu][s];
+        if (2 * lw + sl == s && G.re[mu][s2] + G.im[mu][s2] < 0) neg |= 1u << mu;
+      }
+  }
 
   doublex4 acc[MT][NTL];
 #pragma unroll
@@ -367,44 +459,128 @@ __global__ __launch_bounds__(256) void k_coarsen_mfma(
 #pragma unroll
     for (int nt = 0; nt < NTL; ++nt) acc[mt][nt] = {0.0, 0.0, 0.0, 0.0};
 
-  for (int s0 = 0; s0 < g.nsite; s0 += CM_SB) {
-    // ---- stage u rows of the SB sites as real and (negated) imaginary planes
-    for (int idx = tid; idx < CM_SB * ROW; idx += 256) {
-      const int s = idx / ROW, r = idx - s * ROW;
-      const int e = r / NB, c = r - e * NB;
-      const bool ok = s0 + s < g.nsite;
-      const int xb = ok ? g.face_site(s0 + s) : 0;
-      const cplx<double> u = basis[((size_t)xc * Vb + xb) * ROW + r];
-      sUr[s][e][c] = ok ? u.re : 0.0;
-      sUi[s][e][c] = ok ? -u.im : 0.0;
+  // block coordinates of this wavefront's site, advanced over the point's
+  // sites (lexicographic over the block, or over the face without coordinate
+  // mu, which stays at the block's last (+mu) or first (-mu) layer)
+  int bc[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) bc[d] = !SELF && d == g.mu && g.disp > 0 ? g.blk.L[d] - 1 : 0;
+  auto advance = [&](int n) __attribute__((always_inline)) {
+    for (int i = 0; i < n; ++i) {
+      int carry = 1;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const bool fixed = !SELF && d == g.mu;
+        const int c = bc[d] + (fixed ? 0 : carry);
+        const bool wrap = !fixed && c == g.blk.L[d];
+        carry = fixed ? carry : wrap ? 1 : 0;
+        bc[d] = wrap ? 0 : c;
+      }
     }
-    // ---- W: wavefront w builds site w of the stage, lane l = (lw, c') with
-    // lw = l / NB (both chiralities in one instruction stream; the u staging
-    // above is not read here, so no barrier separates the two)
-    {
-      const int s = __builtin_amdgcn_readfirstlane(tid >> 6);
-      const int lw = l / NB, cp = l - lw * NB;
-      if (l < 2 * NB) {
-        cplx<double> ws[6], wo[6];
-        if (s0 + s < g.nsite) {
-          coarsen_w_lane<NB, 1>(g, G, g.face_site(s0 + s), lw, cp, ws, wo);
+  };
+  advance(ss);
+
+  for (int s0 = 0; s0 < g.nsite; s0 += SB) {
+    cplx<double> ur[NU], ws[3], wo[3];
+#pragma unroll
+    for (int e = 0; e < 3; ++e) ws[e] = wo[e] = {0.0, 0.0};
+    // (opaque here, or the eight phases would be kept in registers over the loop)
+    asm volatile("" : "+v"(neg));
+    const bool ok = s0 + ss < g.nsite;  // uniform over the wavefront
+    if (ok) {
+      int xb = 0, x = 0;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        xb += bc[d] * g.bs[d];
+        x += (g.cc[d] * g.blk.L[d] + bc[d]) * g.fs[d];
+      }
+      xb = __builtin_amdgcn_readfirstlane(xb);
+      x = __builtin_amdgcn_readfirstlane(x);
+      const cplx<double>* ub = basis + ((size_t)xc * Vb + xb) * ROW;
+#pragma unroll
+      for (int q = 0; q < NU; ++q) ur[q] = ub[min(li + q * LPS, ROW - 1)];
+      auto hop = [&](auto qc) __attribute__((always_inline)) {
+        constexpr int q = decltype(qc)::value, qm = q & 3, disp = q < 4 ? 1 : -1;
+        const bool inner = (unsigned)(bc[qm] + disp) < (unsigned)g.blk.L[qm];
+        // self: inner hops, by the reference's coordinate mask (x_mu mod b !=
+        // b-1 for +mu, != 0 for -mu)
+        if (!(SELF ? inner : q == p)) return;  // uniform over the wavefront
+        // fine neighbour y = x + disp*mu (periodic) and its panel row
+        const int fq = g.cc[qm] * g.blk.L[qm] + bc[qm] + disp;
+        const int y = x + disp * g.fs[qm] -
+                      (fq < 0 ? -g.fine.L[qm] * g.fs[qm]
+                              : fq >= g.fine.L[qm] ? g.fine.L[qm] * g.fs[qm] : 0);
+        int ry;
+        if (inner) {
+          ry = xc * Vb + xb + disp * g.bs[qm];
         } else {
-#pragma unroll
-          for (int e = 0; e < 6; ++e) ws[e] = wo[e] = {0.0, 0.0};
+          const int cq = g.cc[qm] + disp;
+          const int xn = xc + disp * g.cs[qm] -
+                         (cq < 0 ? -g.coarse.L[qm] * g.cs[qm]
+                                 : cq >= g.coarse.L[qm] ? g.coarse.L[qm] * g.cs[qm] : 0);
+          ry = xn * Vb + xb - disp * (g.blk.L[qm] - 1) * g.bs[qm];
         }
+        const int lsite = __builtin_amdgcn_readfirstlane(q < 4 ? x : y);
+        const scalar_f64_ptr U =
+            (scalar_f64_ptr)(uintptr_t)(gauge + ((size_t)qm * Vf + lsite) * 9);
+        const cplx<double>* uy = basis + (size_t)__builtin_amdgcn_readfirstlane(ry) * ROW +
+                                 (size_t)e0 * NB + cp;
+        cplx<double> B[3];
 #pragma unroll
-        for (int e = 0; e < 6; ++e) {
-          sWr[s][lw][6 * lw + e][cp] = ws[e].re;
-          sWi[s][lw][6 * lw + e][cp] = ws[e].im;
-          sWr[s][lw][6 - 6 * lw + e][cp] = wo[e].re;
-          sWi[s][lw][6 - 6 * lw + e][cp] = wo[e].im;
+        for (int k = 0; k < 3; ++k) B[k] = uy[k * NB];
+        coarsen_hop<q>(neg, U, B, ws, wo);
+      };
+      // g_x and g_y exchange the spins of a chirality: their images belong to
+      // the other lane of the pair
+      hop(std::integral_constant<int, 0>{});
+      hop(std::integral_constant<int, 1>{});
+      hop(std::integral_constant<int, 4>{});
+      hop(std::integral_constant<int, 5>{});
+#pragma unroll
+      for (int e = 0; e < 3; ++e) wo[e] = {swap_pair(wo[e].re), swap_pair(wo[e].im)};
+      hop(std::integral_constant<int, 2>{});
+      hop(std::integral_constant<int, 3>{});
+      hop(std::integral_constant<int, 6>{});
+      hop(std::integral_constant<int, 7>{});
+      if constexpr (SELF) {  // diagonal (mass + clover) term, block-diagonal in chirality
+        const cplx<double>* D = diag + ((size_t)x * 2 + lw) * 36 + 18 * sl;
+        const cplx<double>* ux = ub + (size_t)(6 * lw) * NB + cp;
+#pragma unroll
+        for (int b = 0; b < 6; ++b) {
+          const cplx<double> vb = ux[b * NB];
+#pragma unroll
+          for (int r = 0; r < 3; ++r) cmac(ws[r], D[r * 6 + b], vb);
         }
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < NU; ++q) ur[q] = {0.0, 0.0};
+    }
+    advance(SB);
+    __syncthreads();  // the previous stage's products have been read
+#pragma unroll
+    for (int q = 0; q < NU; ++q) {
+      const int r = li + q * LPS, e = r / NB, c = r - e * NB;
+      if (ROW % LPS == 0 || r < ROW) {
+        sUr[(ss * 12 + e) * NBP + c] = ur[q].re;
+        sUi[(ss * 12 + e) * NBP + c] = -ur[q].im;
+      }
+    }
+    if (col) {
+      const int base = (ss * 2 + lw) * 12 * NBP + cp;
+#pragma unroll
+      for (int e = 0; e < 3; ++e) {
+        sWr[base + (e0 + e) * NBP] = ws[e].re;
+        sWi[base + (e0 + e) * NBP] = ws[e].im;
+        const int eo = 6 - 6 * lw + 3 * sl + e;
+        sWr[base + eo * NBP] = wo[e].re;
+        sWi[base + eo * NBP] = wo[e].im;
       }
     }
     __syncthreads();
     // ---- the block's GEMM: per site three k-steps of two elements each
 #pragma unroll 1
-    for (int s = 0; s < CM_SB; ++s)
+    for (int s = 0; s < SB; ++s)
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         const int e = 6 * kb + 2 * q + (lk >> 1);  // element of this lane's K slot
@@ -427,17 +603,15 @@ __global__ __launch_bounds__(256) void k_coarsen_mfma(
           for (int nt = 0; nt < NTL; ++nt)
             acc[mt][nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[mt], b[nt], acc[mt][nt], 0, 0, 0);
       }
-    __syncthreads();
   }
   // ---- write A_p(xc) rows k*NB + c, columns l*NB + c' (component v)
   constexpr int N = 2 * NB;
-  double* Ap = reinterpret_cast<double*>(links + ((size_t)g.p * Vc + xc) * N * N);
+  double* Ap = reinterpret_cast<double*>(links + ((size_t)p * Vc + xc) * N * N);
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int nt = 0; nt < NTL; ++nt) {
-      const int n = nt * 16 + (l & 15);
-      const int cq = n >> 1;
+      const int cq = (nt * 16 + (l & 15)) >> 1;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int c = mt * 16 + 4 * r + lk;
@@ -486,9 +660,14 @@ static void launch_coarsen_t(const mgc_aggregation* agg, const mgc_fine_op* fop,
 template <int NB>
 static void launch_coarsen_mfma_t(const mgc_aggregation* agg, const mgc_fine_op* fop,
                                   const int* plist, int np, cplx<double>* links, hipStream_t s) {
-  k_coarsen_mfma<NB><<<agg->Vc * np, 256, 0, s>>>(agg->basis64, fop->gauge64, fop->diag64,
-                                                  agg->fine, agg->coarse, agg->blk, agg->Vf,
-                                                  agg->Vb, plist, np, agg->Vc, links);
+  // the faces (all points of the list but the last, the self point), then the self point
+  k_coarsen_mfma<NB, false><<<agg->Vc * (np - 1), 256, 0, s>>>(
+      agg->basis64, fop->gauge64, fop->diag64, agg->fine, agg->coarse, agg->blk, agg->Vf, agg->Vb,
+      plist, np - 1, agg->Vc, links);
+  MGC_LAUNCH_CHECK();
+  k_coarsen_mfma<NB, true><<<agg->Vc, 256, 0, s>>>(
+      agg->basis64, fop->gauge64, fop->diag64, agg->fine, agg->coarse, agg->blk, agg->Vf, agg->Vb,
+      plist, 1, agg->Vc, links);
   MGC_LAUNCH_CHECK();
 }
 
