@@ -20,19 +20,33 @@ namespace mgc {
 // ---------------------------------------------------------------------------
 // layout conversion
 // ---------------------------------------------------------------------------
-__global__ void k_import_basis(const cplx<double>* __restrict__ src, int nb, int Vf, int Ef,
-                               size_t total, const int* __restrict__ blk_fine,
-                               cplx<double>* __restrict__ dst) {
-  size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  for (; t < total; t += stride) {
-    const int i = (int)(t % nb);
-    size_t r = t / nb;
-    const int e = (int)(r % Ef);
-    r /= Ef;  // r = xc*Vb + xb
-    const int sf = blk_fine[r];
-    dst[t] = src[((size_t)i * Vf + sf) * Ef + e];
+// Basis vectors [i][site][e] to panels [row][i] (row = (block, block site, e)),
+// IB_ROWS panel rows a workgroup through LDS: a thread keeps its row and reads
+// it of every IB_ROWS-th vector (runs of whole sites, 768 bytes where a block
+// is four sites wide), and the tile leaves as one contiguous run.  A copy bound
+// by HBM: 32^4, nb 32 (12.9 GB) 2.46 ms (5.2 TB/s), 4.3 ms with the panel order
+// on both sides.
+constexpr int IB_ROWS = 48, IB_THREADS = 192;
+__global__ __launch_bounds__(IB_THREADS) void k_import_basis(
+    const cplx<double>* __restrict__ src, int nb, int Vf, int Ef, size_t rows,
+    const int* __restrict__ blk_fine, cplx<double>* __restrict__ dst) {
+  extern __shared__ unsigned char smem_raw[];
+  cplx<double>* s_t = reinterpret_cast<cplx<double>*>(smem_raw);  // [IB_ROWS][nb + 1]
+  const size_t q0 = (size_t)blockIdx.x * IB_ROWS;
+  const int n = (int)(rows - q0 < (size_t)IB_ROWS ? rows - q0 : (size_t)IB_ROWS);
+  const int r = threadIdx.x % IB_ROWS;
+  if (r < n) {
+    const size_t q = q0 + r;
+    const int e = (int)(q % Ef);
+    const cplx<double>* p = src + (size_t)blk_fine[q / Ef] * Ef + e;
+    const size_t vec = (size_t)Vf * Ef;
+#pragma unroll 4
+    for (int i = threadIdx.x / IB_ROWS; i < nb; i += IB_THREADS / IB_ROWS)
+      s_t[r * (nb + 1) + i] = p[i * vec];
   }
+  __syncthreads();
+  for (int t = threadIdx.x; t < n * nb; t += IB_THREADS)
+    dst[q0 * nb + t] = s_t[t + t / nb];  // row t / nb of pitch nb + 1
 }
 
 __global__ void k_export_basis(const cplx<double>* __restrict__ src, int nb, int Vf, int Ef,
@@ -1120,10 +1134,11 @@ int mgc_aggregation_info(const mgc_aggregation* a, int coarse_dims[4], int* nb, 
 int mgc_aggregation_set_basis(mgc_aggregation* a, const void* basis_f64, void* stream) {
   return guarded([&] {
     MGC_CHECK(a && basis_f64, MGC_ERR_ARG, "null argument");
-    const size_t total = (size_t)a->Vf * a->Ef * a->nb;
+    const size_t rows = (size_t)a->Vf * a->Ef;
     hipStream_t s = as_stream(stream);
-    k_import_basis<<<grid_for(total, 256, 16384), 256, 0, s>>>(
-        (const cplx<double>*)basis_f64, a->nb, a->Vf, a->Ef, total, a->blk_fine, a->basis64);
+    k_import_basis<<<(unsigned)((rows + IB_ROWS - 1) / IB_ROWS), IB_THREADS,
+                     (size_t)IB_ROWS * (a->nb + 1) * sizeof(cplx<double>), s>>>(
+        (const cplx<double>*)basis_f64, a->nb, a->Vf, a->Ef, rows, a->blk_fine, a->basis64);
     MGC_LAUNCH_CHECK();
     a->basis_set = true;
     a->basis32_valid = false;

@@ -1,0 +1,59 @@
+"""Exact round trips through the tiled layout conversions: links (32 x 32 tiles,
+both external layouts) and basis (48 panel rows a tile), at sizes with partial
+tiles.  Values are moved, not computed: equality bit for bit (FP32 operators:
+equality with the rounded input)."""
+import numpy as np
+import pytest
+
+import oracle
+from helpers import gauss, rand_links
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("N", [2, 30, 32, 34, 64, 66])
+def test_links_round_trip(gpu, N, prec):
+    print(f"[case] links N={N} prec={prec}", flush=True)
+    dims = (2, 1, 3, 2)
+    V = int(np.prod(dims))
+    links = rand_links(dims, N)
+    op = gpu.CoarseOp(dims, N, prec)
+    op.set_links(gpu.DeviceBuffer.from_numpy(links), gpu.LAYOUT_FLAT, invert=False)
+    want = links.reshape(9, V, N, N)
+    if prec == 1:
+        want = want.astype(np.complex64).astype(np.complex128)
+    out = gpu.DeviceBuffer(links.nbytes)
+    op.get_links(out, gpu.LAYOUT_FLAT)
+    gpu.synchronize()
+    assert np.array_equal(out.to_numpy(np.complex128, want.shape), want)
+    op.get_links(out, gpu.LAYOUT_SPLIT)
+    gpu.synchronize()
+    got = out.to_numpy(np.complex128, (9, V, 2, 2, N // 2, N // 2))
+    split = want.reshape(9, V, 2, N // 2, 2, N // 2).transpose(0, 1, 2, 4, 3, 5)
+    assert np.array_equal(got, split)
+
+
+@pytest.mark.parametrize("fd,blk,nb,Ef", [((2, 3, 1, 1), (1, 3, 1, 1), 1, 2),
+                                          ((4, 4, 2, 2), (2, 2, 2, 1), 17, 12),
+                                          ((6, 3, 3, 3), (3, 3, 3, 3), 33, 26),
+                                          ((4, 2, 2, 2), (2, 2, 1, 2), 64, 12)])
+def test_basis_round_trip(gpu, fd, blk, nb, Ef):
+    print(f"[case] basis fd={fd} blk={blk} nb={nb} Ef={Ef}", flush=True)
+    Vf = int(np.prod(fd))
+    B = gauss(nb * Vf * Ef, 821).reshape(nb, Vf, Ef)
+    agg = gpu.Aggregation(fd, blk, nb, Ef)
+    agg.set_basis(gpu.DeviceBuffer.from_numpy(B))
+    out = gpu.DeviceBuffer(B.nbytes)
+    agg.get_basis(out)
+    gpu.synchronize()
+    assert np.array_equal(out.to_numpy(np.complex128, B.shape), B)
+    # the panels themselves: a projection reads them in their own order
+    f = gauss(Vf * Ef, 822).reshape(Vf, Ef)
+    Vc = int(np.prod(oracle.coarse_dims(fd, blk)))
+    oc = gpu.DeviceBuffer(Vc * 2 * nb * 16)
+    agg.project(gpu.DeviceBuffer.from_numpy(f), oc, 0, 1)
+    gpu.synchronize()
+    ref = oracle.project_ef(fd, blk, nb, Ef, B, f)
+    got = oc.to_numpy(np.complex128, (Vc, 2 * nb))
+    assert np.linalg.norm(got - ref) < 1e-13 * np.linalg.norm(ref)
