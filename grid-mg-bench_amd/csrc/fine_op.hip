@@ -314,40 +314,46 @@ __device__ __forceinline__ void wilson_hop_apply(cplx<R>* acc, const GammaTab& G
 // s * 3 + c.  Every element gets the same updates in the same order as in
 // wilson_diag_apply and wilson_hop_apply, so the results are bit-identical;
 // c is uniform over a wavefront, so the tests on it are scalar branches.
-template <typename R, typename DK, typename SP>
-__device__ __forceinline__ void wilson_diag_apply_row(cplx<R>* acc, int c, DK&& dk, SP&& sp) {
-  const int e0 = c, e1 = 3 + c;  // this thread's elements of each block
+// dk[row][b]: packed entry of (row element, b) of block l, the diagonal pair at
+// b = the row's own element; the row elements of a block are c and 3 + c.
+template <typename R>
+__device__ __forceinline__ void wilson_diag_load_row(cplx<R> (&dk)[2][6], int c, int l,
+                                                     const cplx<R>* __restrict__ diag, int x,
+                                                     int sv) {
 #pragma unroll
-  for (int l = 0; l < 2; ++l) {
-    cplx<R>& A0 = acc[2 * l];
-    cplx<R>& A1 = acc[2 * l + 1];
-    cplx<R> v[6];
+  for (int r = 0; r < 2; ++r) {
+    const int e = 3 * r + c;
 #pragma unroll
-    for (int b = 0; b < 6; ++b) v[b] = sp(6 * l + b);
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const bool lo0 = 2 * a == e0, hi0 = 2 * a + 1 == e0;
-      const bool lo1 = 2 * a == e1, hi1 = 2 * a + 1 == e1;
-      if (!(lo0 || hi0 || lo1 || hi1)) continue;
-      const cplx<R> dd = dk(l, a);
-      if (lo0) { A0.re += dd.re * v[2 * a].re; A0.im += dd.re * v[2 * a].im; }
-      if (hi0) { A0.re += dd.im * v[2 * a + 1].re; A0.im += dd.im * v[2 * a + 1].im; }
-      if (lo1) { A1.re += dd.re * v[2 * a].re; A1.im += dd.re * v[2 * a].im; }
-      if (hi1) { A1.re += dd.im * v[2 * a + 1].re; A1.im += dd.im * v[2 * a + 1].im; }
+    for (int b = 0; b < 6; ++b) {
+      const int lo = min(e, b), hi = max(e, b);
+      const int slot = lo == hi ? e / 2 : 3 + lo * (11 - lo) / 2 + hi - lo - 1;
+      dk[r][b] = diag[((size_t)l * 18 + slot) * sv + x];
     }
-    int slot = 3;
+  }
+}
+template <typename R, typename SP>
+__device__ __forceinline__ void wilson_diag_apply_row(cplx<R>* acc, int c,
+                                                      const cplx<R> (&dk)[2][6], int l, SP&& sp) {
+  cplx<R> v[6];
 #pragma unroll
-    for (int a = 0; a < 6; ++a)
+  for (int b = 0; b < 6; ++b) v[b] = sp(6 * l + b);
 #pragma unroll
-      for (int b = a + 1; b < 6; ++b, ++slot) {
-        const bool u0 = a == e0, u1 = a == e1, w0 = b == e0, w1 = b == e1;
-        if (!(u0 || u1 || w0 || w1)) continue;
-        const cplx<R> u = dk(l, slot);
-        if (u0) cmac(A0, u, v[b]);
-        if (u1) cmac(A1, u, v[b]);
-        if (w0) cmac_conj(A0, u, v[a]);
-        if (w1) cmac_conj(A1, u, v[a]);
+  for (int r = 0; r < 2; ++r) {
+    cplx<R>& A = acc[2 * l + r];
+    const int e = 3 * r + c;
+#pragma unroll
+    for (int b = 3 * r; b < 3 * r + 3; ++b)
+      if (b == e) {
+        const R d = b % 2 ? dk[r][b].im : dk[r][b].re;
+        A.re += d * v[b].re;
+        A.im += d * v[b].im;
       }
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      if (b == e) continue;
+      if (b > e) cmac(A, dk[r][b], v[b]);   // upper: D_eb v_b
+      else cmac_conj(A, dk[r][b], v[b]);    // lower: conj(D_be) v_b
+    }
   }
 }
 // lk(j): entry j of row c of U_mu(x) (p < 4) or of column c of U_mu(y)
@@ -579,20 +585,25 @@ __global__ __launch_bounds__(256) void k_wilson_lds(const cplx<R>* __restrict__ 
 // rhs's thread.  The self stage's "link" is clover slots 0..8 of block 0.
 // Record layout, output path and per-thread arithmetic are those of
 // k_wilson_lds.
-template <typename R, int LPT>
+// Which site, rhs and chunk a thread copies is the same in every stage: the
+// divisions by nrhs are done once and their results kept, one register a chunk,
+// and the neighbour sites are kept as 32-bit chunk indexes too.  With the divisions in each stage the
+// integer multiplies took twice the time of the FP32 arithmetic: 12 rhs at 32^4
+// 1.42 ms.
+template <typename R, int LPT, bool DAG>
 __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U,
                                                    const cplx<R>* __restrict__ diag,
                                                    const cplx<R>* __restrict__ in,
                                                    cplx<R>* __restrict__ out,
                                                    const int* __restrict__ nbr, int V, int sv,
-                                                   int nrhs, unsigned mask, int dag,
-                                                   WilsonTiles wt) {
+                                                   int nrhs, unsigned mask, WilsonTiles wt) {
   constexpr int CPS = 12 * (int)sizeof(cplx<R>) / 16;
   constexpr int RS = CPS + 1;
   constexpr int SMAX = LPT == 1 ? 28 : 51;  // sites per tile at nrhs >= 9 or >= 5
   __shared__ uint4 s_rec[256 * RS];
   __shared__ cplx<R> s_lk[9 * SMAX];  // [k][site]
   __shared__ int s_nb[9][SMAX];       // [hop][site], hop 8 = the site itself
+  __shared__ unsigned s_first[9][SMAX];  // first 16-byte chunk of that site's records
   const int T = (int)blockDim.x;
   const int S = T / nrhs;
   const int t = (int)threadIdx.x;
@@ -604,9 +615,29 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
 
   for (int j = t; j < 8 * S; j += T) {  // j = s * 8 + h: consecutive lanes, consecutive entries
     const int s = j >> 3, h = j & 7;
-    s_nb[h][s] = x0 + s < V ? nbr[(size_t)(x0 + s) * 8 + h] : 0;
+    const int y = x0 + s < V ? nbr[(size_t)(x0 + s) * 8 + h] : 0;
+    s_nb[h][s] = y;
+    s_first[h][s] = (unsigned)y * (unsigned)(nrhs * CPS);
   }
-  if (t < S) s_nb[8][t] = x0 + t < V ? x0 + t : 0;
+  if (t < S) {
+    const int y = x0 + t < V ? x0 + t : 0;
+    s_nb[8][t] = y;
+    s_first[8][t] = (unsigned)y * (unsigned)(nrhs * CPS);
+  }
+  // chunk c = t + k*T of the tile's records: site slot (6 bits) and chunk of
+  // that site's records; link entry j = t + m*T: site slot and element offset
+  unsigned chunk[CPS], lslot[LPT], loff[LPT];
+#pragma unroll
+  for (int k = 0; k < CPS; ++k) {
+    const int c = t + k * T, s = c / (CPS * nrhs);
+    chunk[k] = (unsigned)(c - s * (CPS * nrhs)) << 6 | (unsigned)s;
+  }
+#pragma unroll
+  for (int m = 0; m < LPT; ++m) {
+    const int j = t + m * T, k = j / S;
+    lslot[m] = (unsigned)(j - k * S);
+    loff[m] = (unsigned)k * (unsigned)sv;
+  }
   auto next_hop = [&](int i) {
     for (int k = i + 1; k < 9; ++k) {
       const int h = k == 0 ? 8 : k - 1;
@@ -622,28 +653,24 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
   u32x4 nrec[CPS];
   cplx<R> nlk[LPT];
   // loads of hop h into registers: record chunks c = t + k*T of the tile's
-  // records, and link entries j = t + m*T (k = j / S, site j % S) for j < 9 S
+  // records, and link entries j = t + m*T (element j / S, site j % S) for j < 9 S
   auto issue = [&](int h) {
 #pragma unroll
     for (int k = 0; k < CPS; ++k) {
-      const int c = t + k * T, q = c / CPS, e = c - q * CPS, s = q / nrhs, r = q - s * nrhs;
-      nrec[k] = in4[((size_t)s_nb[h][s] * nrhs + r) * CPS + e];
+      nrec[k] = in4[s_first[h][chunk[k] & 63] + (chunk[k] >> 6)];
     }
 #pragma unroll
     for (int m = 0; m < LPT; ++m) {
-      const int j = t + m * T;
-      if (j < 9 * S) {
-        const int k = j / S, s = j - k * S;
-        const cplx<R>* u = h == 8 ? diag + s_nb[8][s]
-                                  : U + (size_t)(h & 3) * 9 * sv + (h < 4 ? s_nb[8][s] : s_nb[h][s]);
-        nlk[m] = u[(size_t)k * sv];
+      if (t + m * T < 9 * S) {
+        const cplx<R>* u = h == 8 ? diag : U + (size_t)(h & 3) * 9 * sv;
+        nlk[m] = u[loff[m] + (unsigned)s_nb[h < 4 ? 8 : h][lslot[m]]];
       }
     }
   };
   auto rec = [&](int e) {
     cplx<R> v = reinterpret_cast<const cplx<R>*>(&s_rec[rec_pos<CPS, RS>(t, e * CPS / 12)])
         [(e * CPS) % 12 / 6];
-    if (dag && e >= 6) { v.re = -v.re; v.im = -v.im; }
+    if (DAG && e >= 6) { v.re = -v.re; v.im = -v.im; }
     return v;
   };
 
@@ -683,15 +710,16 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
 #pragma unroll
   for (int e = 0; e < 12; ++e) {
     cplx<R> v = acc[e];
-    if (dag && e >= 6) { v.re = -v.re; v.im = -v.im; }
+    if (DAG && e >= 6) { v.re = -v.re; v.im = -v.im; }
     reinterpret_cast<cplx<R>*>(&s_rec[rec_pos<CPS, RS>(t, e * CPS / 12)])[(e * CPS) % 12 / 6] = v;
   }
   __syncthreads();
   uint4* out4 = reinterpret_cast<uint4*>(out);
 #pragma unroll
   for (int k = 0; k < CPS; ++k) {
-    const int c = t + k * T, q = c / CPS, e = c - q * CPS, s = q / nrhs, r = q - s * nrhs;
-    if (x0 + s < V) out4[((size_t)(x0 + s) * nrhs + r) * CPS + e] = s_rec[rec_pos<CPS, RS>(q, e)];
+    const int c = t + k * T, s = (int)(chunk[k] & 63);
+    if (x0 + s < V)
+      out4[(size_t)x0 * (nrhs * CPS) + c] = s_rec[rec_pos<CPS, RS>(c / CPS, c % CPS)];
   }
 }
 
@@ -700,106 +728,116 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
 // keeps 4 accumulators instead of 12 and loads one row (or column) of each
 // hop's link instead of all nine entries, so it needs far fewer registers
 // than k_wilson_lds's thread per site, and more wavefronts fit on a SIMD.
-// The records are staged in LDS as in k_wilson_lds (each read by the three
-// threads of the site); hops run self first, then 0..7, with the next hop's
-// neighbour sites staged one hop ahead and the link loads issued before the
-// record copy.
-template <typename R>
+// The tile's 8 x 64 neighbour sites are read once into LDS, together with the
+// self records and the clover entries of the row.  Hops run
+// self first, then 0..7; each stage's records are staged in LDS (each read by
+// the three threads of the site), the next stage's loads issued before its
+// arithmetic.
+// What bounds it: HBM traffic is the algorithmic one (48^4 FP64: 6.8 GB read, 1.0
+// written); the rest is latency, so the loads that do not depend on others are
+// issued together.  48^4 FP64 2.19 -> 2.08 ms, 32^4 FP32 0.233 -> 0.206, 16^4 FP32
+// 20.6 -> 13.4 us against one stage's loads at a time (neighbour sites one hop
+// ahead, clover entries during their arithmetic).  Two hops a stage: 0.257 ms at
+// 32^4 FP32, for the occupancy that the second buffer takes.
+template <typename R, bool DAG>
 __global__ __launch_bounds__(192) void k_wilson_row(const cplx<R>* __restrict__ U,
                                                     const cplx<R>* __restrict__ diag,
                                                     const cplx<R>* __restrict__ in,
                                                     cplx<R>* __restrict__ out,
                                                     const int* __restrict__ nbr, int V, int sv,
-                                                    unsigned mask, int dag, WilsonTiles wt) {
+                                                    unsigned mask, WilsonTiles wt) {
   constexpr int CPS = 12 * (int)sizeof(cplx<R>) / 16;
   constexpr int RS = CPS + 1;
   constexpr int S = 64, T = 192, NCH = S * CPS / T;  // record chunks per thread
   static_assert(S * CPS % T == 0, "whole chunks per thread");
-  __shared__ uint4 s_rec[S * RS];
-  __shared__ int s_y[2][S];
+  // native 4-vectors: copies of uint4 (a union type) are memcpys that keep
+  // a staging array out of registers
+  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  __shared__ u32x4 s_rec[S * RS];
+  __shared__ int s_nb[8][S];
   const int t = (int)threadIdx.x;
   const int c = __builtin_amdgcn_readfirstlane(t >> 6);  // colour row of this wavefront
   const int sl = t & 63;
   const int x0 = wilson_tile_site(wt, (int)blockIdx.x);
-  const int x = x0 + sl;
-  const bool live = x < V;
+  const bool live = x0 + sl < V;
+  const int x = live ? x0 + sl : 0;  // past the lattice: site 0, whose result is not stored
   const GammaTab G = gamma_table();
-
-  auto hop_site = [&](int s, int h) {  // h = 8: the site itself
-    const int xs = x0 + s;
-    if (xs >= V) return 0;
-    return h == 8 ? xs : nbr[(size_t)xs * 8 + h];
-  };
-  auto next_hop = [&](int i) {
-    for (int k = i + 1; k < 9; ++k) {
-      const int h = k == 0 ? 8 : k - 1;
-      if ((mask >> h) & 1u) return h;
-    }
-    return -1;
-  };
-  const uint4* in4 = reinterpret_cast<const uint4*>(in);
+  const u32x4* in4 = reinterpret_cast<const u32x4*>(in);
+  auto on = [&](int h) { return ((mask >> h) & 1u) != 0; };
   auto rec = [&](int e) {  // element e of this site's staged record
     cplx<R> v = reinterpret_cast<const cplx<R>*>(&s_rec[rec_pos<CPS, RS>(sl, e * CPS / 12)])
         [(e * CPS) % 12 / 6];
-    if (dag && e >= 6) { v.re = -v.re; v.im = -v.im; }
+    if (DAG && e >= 6) { v.re = -v.re; v.im = -v.im; }
     return v;
   };
-
-  cplx<R> acc[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) acc[e] = {R(0), R(0)};
-  int cb = 0;
-  const int h0 = next_hop(-1);
-  if (h0 >= 0) {
-    if (t < S) s_y[0][t] = hop_site(t, h0);
-    __syncthreads();
-  }
-  cplx<R> lk[3];
-  // one stage's loads: this hop's link row (or column), then the records of
-  // its neighbour sites into LDS, the next hop's sites staged one ahead
-  auto begin_stage = [&](int h, int hn) __attribute__((always_inline)) {
-    __syncthreads();  // every thread is done with the previous hop's records
-    const int y = s_y[cb][sl];
-    if (live && h != 8) {
-      const cplx<R>* u = U + (size_t)(h & 3) * 9 * sv + (h < 4 ? x : y);
-#pragma unroll
-      for (int j = 0; j < 3; ++j) lk[j] = u[(size_t)(h < 4 ? c * 3 + j : j * 3 + c) * sv];
-    }
-    const int ynext = hn >= 0 && t < S ? hop_site(t, hn) : 0;
+  u32x4 nrec[NCH];
+  cplx<R> nlk[3];
+  auto issue = [&](int h) __attribute__((always_inline)) {
+    if (!on(h)) return;
 #pragma unroll
     for (int k = 0; k < NCH; ++k) {
       const int cc = t + k * T, q = cc / CPS, e = cc - q * CPS;
-      s_rec[rec_pos<CPS, RS>(q, e)] = in4[(size_t)s_y[cb][q] * CPS + e];
+      const int y = h == 8 ? (x0 + q < V ? x0 + q : 0) : s_nb[h][q];
+      nrec[k] = in4[(size_t)y * CPS + e];
     }
-    if (hn >= 0 && t < S) s_y[cb ^ 1][t] = ynext;
-    __syncthreads();
-    cb ^= 1;
+    if (h != 8) {
+      const cplx<R>* u = U + (size_t)(h & 3) * 9 * sv + (h < 4 ? x : s_nb[h][sl]);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) nlk[j] = u[(size_t)(h < 4 ? c * 3 + j : j * 3 + c) * sv];
+    }
   };
-  // the self stage apart from the hop loop, so that the loop body stays
-  // small enough to be unrolled (every hop index a compile-time constant)
-  if ((mask >> 8) & 1u) {
-    begin_stage(8, next_hop(0));
-    if (live)
-      wilson_diag_apply_row<R>(acc, c, [&](int l, int s) {
-        return diag[((size_t)l * 18 + s) * sv + x];
-      }, rec);
-  }
+  auto stage = [&](int h) __attribute__((always_inline)) {
+    if (!on(h)) return;
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) {
+      const int cc = t + k * T;
+      s_rec[rec_pos<CPS, RS>(cc / CPS, cc % CPS)] = nrec[k];
+    }
+  };
+
+  i32x4 nb4 = {0, 0, 0, 0};
+  if (t < 2 * S && x0 + (t >> 1) < V)
+    nb4 = reinterpret_cast<const i32x4*>(nbr)[(size_t)x0 * 2 + t];
+  issue(8);
+  cplx<R> dk[2][2][6];
+  if (on(8))
+#pragma unroll
+    for (int l = 0; l < 2; ++l) wilson_diag_load_row<R>(dk[l], c, l, diag, x, sv);
+  if (t < 2 * S)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s_nb[(t & 1) * 4 + k][t >> 1] = nb4[k];
+  stage(8);
+  cplx<R> acc[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = {R(0), R(0)};
+  __syncthreads();  // s_nb and the self records
+  issue(0);
+  if (on(8))
+#pragma unroll
+    for (int l = 0; l < 2; ++l) wilson_diag_apply_row<R>(acc, c, dk[l], l, rec);
 #pragma unroll
   for (int p = 0; p < 8; ++p) {
-    if (!((mask >> p) & 1u)) continue;
-    begin_stage(p, next_hop(p + 1));
-    if (live) wilson_hop_apply_row<R>(acc, G, p, [&](int j) { return lk[j]; }, rec);
+    if (!on(p) && !(p < 7 && on(p + 1))) continue;
+    __syncthreads();  // every thread is done with the previous stage's records
+    stage(p);
+    cplx<R> lk[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) lk[j] = nlk[j];
+    if (p < 7) issue(p + 1);
+    __syncthreads();
+    if (on(p)) wilson_hop_apply_row<R>(acc, G, p, [&](int j) { return lk[j]; }, rec);
   }
   __syncthreads();
 #pragma unroll
   for (int s = 0; s < 4; ++s) {
     const int e = s * 3 + c;
     cplx<R> v = acc[s];
-    if (dag && s >= 2) { v.re = -v.re; v.im = -v.im; }
+    if (DAG && s >= 2) { v.re = -v.re; v.im = -v.im; }
     reinterpret_cast<cplx<R>*>(&s_rec[rec_pos<CPS, RS>(sl, e * CPS / 12)])[(e * CPS) % 12 / 6] = v;
   }
   __syncthreads();
-  uint4* out4 = reinterpret_cast<uint4*>(out);
+  u32x4* out4 = reinterpret_cast<u32x4*>(out);
 #pragma unroll
   for (int k = 0; k < NCH; ++k) {
     const int cc = t + k * T, q = cc / CPS, e = cc - q * CPS;
@@ -926,9 +964,9 @@ static void fine_apply(mgc_fine_op* op, const void* in, void* out, int prec, int
   const WilsonTiles wr = wilson_tiles_fixed(op->lat, 64);
   const unsigned gr = (unsigned)((op->V + 63) / 64);
   if (prec == MGC_F64 && wilson_row(nrhs)) {
-    k_wilson_row<double><<<gr, 192, 0, s>>>(op->gsoa64, op->dsoa64, (const cplx<double>*)in,
-                                            (cplx<double>*)out, op->nbr, op->V, op->sv, mask,
-                                            dag, wr);
+    auto k = dag ? k_wilson_row<double, true> : k_wilson_row<double, false>;
+    k<<<gr, 192, 0, s>>>(op->gsoa64, op->dsoa64, (const cplx<double>*)in, (cplx<double>*)out,
+                         op->nbr, op->V, op->sv, mask, wr);
   } else if (prec == MGC_F64) {
     auto k = lds ? k_wilson_lds<double> : k_wilson<double>;
     k<<<g, threads, 0, s>>>(op->gsoa64, op->dsoa64, (const cplx<double>*)in, (cplx<double>*)out,
@@ -950,19 +988,23 @@ static void fine_apply(mgc_fine_op* op, const void* in, void* out, int prec, int
       op->gsoa32 = g32;
       op->dsoa32 = d32;
     }
+    const cplx<float>* v = (const cplx<float>*)in;
+    cplx<float>* o = (cplx<float>*)out;
+    // k_wilson_pf keeps chunk indexes of the field in 32 bits
+    const bool pf = g_wilson_variant != 1 && nrhs >= 5 &&
+                    (size_t)op->V * nrhs * 6 <= (size_t)UINT32_MAX;
     if (wilson_row(nrhs)) {
-      k_wilson_row<float><<<gr, 192, 0, s>>>(op->gsoa32, op->dsoa32, (const cplx<float>*)in,
-                                             (cplx<float>*)out, op->nbr, op->V, op->sv, mask,
-                                             dag, wr);
-      MGC_LAUNCH_CHECK();
-      return;
+      auto k = dag ? k_wilson_row<float, true> : k_wilson_row<float, false>;
+      k<<<gr, 192, 0, s>>>(op->gsoa32, op->dsoa32, v, o, op->nbr, op->V, op->sv, mask, wr);
+    } else if (lds && pf) {
+      auto k = nrhs >= 9 ? (dag ? k_wilson_pf<float, 1, true> : k_wilson_pf<float, 1, false>)
+                         : (dag ? k_wilson_pf<float, 2, true> : k_wilson_pf<float, 2, false>);
+      k<<<g, threads, 0, s>>>(op->gsoa32, op->dsoa32, v, o, op->nbr, op->V, op->sv, nrhs, mask, wt);
+    } else {
+      auto k = lds ? k_wilson_lds<float> : k_wilson<float>;
+      k<<<g, threads, 0, s>>>(op->gsoa32, op->dsoa32, v, o, op->nbr, op->V, op->sv, nrhs, mask,
+                              dag, wt);
     }
-    auto k = !lds ? k_wilson<float>
-             : g_wilson_variant == 1 || nrhs < 5 ? k_wilson_lds<float>
-             : nrhs >= 9                        ? k_wilson_pf<float, 1>
-                                                : k_wilson_pf<float, 2>;
-    k<<<g, threads, 0, s>>>(op->gsoa32, op->dsoa32, (const cplx<float>*)in, (cplx<float>*)out,
-                            op->nbr, op->V, op->sv, nrhs, mask, dag, wt);
   } else {
     throw Error(MGC_ERR_PRECISION, "fine operator: F64 or F32");
   }
