@@ -446,17 +446,36 @@ __device__ __forceinline__ int rec_pos(int q, int e) {
   static_assert(RS > CPS, "padded records");
   return q * RS + e;
 }
+// Chunk c (< 4096) of a tile's records, CPS of them a record and a site's nrhs
+// records contiguous: its site slot s, its chunk among the site's (c - s *
+// nrhs * CPS) and its LDS position.  No integer division: (c + 1/2) / (nrhs *
+// CPS) is at least 1/(2 nrhs CPS) >= 1.6e-4 from an integer, the rounding of the
+// quotient (< 256) in FP32 at most 4e-5; c / CPS by a 16-bit reciprocal, exact
+// for c < 8192.  (Quarter-rate integer multiplies of the divisions took as long
+// as the arithmetic.)
+struct WilsonChunk {
+  int s, off, pos;
+};
+template <int CPS, int RS>
+__device__ __forceinline__ WilsonChunk wilson_chunk(int c, int per_site, float inv_per_site) {
+  static_assert((CPS == 6 || CPS == 12) && RS == CPS + 1, "record layout");
+  WilsonChunk w;
+  w.s = (int)(((float)c + 0.5f) * inv_per_site);
+  w.off = c - (int)__umul24(w.s, per_site);
+  w.pos = c + (int)(__umul24(c, CPS == 6 ? 10923 : 5462) >> 16);  // q * RS + e, q = c / CPS
+  return w;
+}
 // Cooperative copy of T records of CPS 16-byte chunks into LDS: chunk
-// c = t + k*T of record q = c / CPS (tile site q / nrhs, rhs q % nrhs), part
-// e = c % CPS, is read from record (sites[q / nrhs], rhs) of the field and
-// stored at position rec_pos(q, e).
+// c = t + k*T of the tile's records is read from the records of site
+// sites[s] and stored at its LDS position.
 template <int CPS, int RS>
 __device__ __forceinline__ void wilson_copy(uint4* s_rec, const uint4* __restrict__ in4,
-                                            const int* sites, int t, int T, int nrhs) {
+                                            const int* sites, int t, int T, int per_site,
+                                            float inv_per_site) {
 #pragma unroll
   for (int k = 0; k < CPS; ++k) {
-    const int c = t + k * T, q = c / CPS, e = c - q * CPS, s = q / nrhs, r = q - s * nrhs;
-    s_rec[rec_pos<CPS, RS>(q, e)] = in4[((size_t)sites[s] * nrhs + r) * CPS + e];
+    const WilsonChunk w = wilson_chunk<CPS, RS>(t + k * T, per_site, inv_per_site);
+    s_rec[w.pos] = in4[(size_t)sites[w.s] * per_site + w.off];
   }
 }
 
@@ -491,6 +510,8 @@ __global__ __launch_bounds__(256) void k_wilson_lds(const cplx<R>* __restrict__ 
   const int x0 = wilson_tile_site(wt, (int)blockIdx.x);
   const int x = x0 + t / nrhs;  // thread t is record t: site t / nrhs, rhs t % nrhs
   const bool live = x < V;
+  const int per_site = nrhs * CPS;
+  const float inv_per_site = 1.0f / (float)per_site;
   const GammaTab G = gamma_table();
 
   auto pos = [&](int q, int e) { return rec_pos<CPS, RS>(q, e); };
@@ -543,7 +564,7 @@ __global__ __launch_bounds__(256) void k_wilson_lds(const cplx<R>* __restrict__ 
       for (int k = 0; k < 9; ++k) lk[k] = u[(size_t)k * sv];
     }
     const int ynext = hn >= 0 && t < S ? hop_site(t, hn) : 0;
-    wilson_copy<CPS, RS>(s_rec, in4, s_y[cb], t, T, nrhs);
+    wilson_copy<CPS, RS>(s_rec, in4, s_y[cb], t, T, per_site, inv_per_site);
     if (hn >= 0 && t < S) s_y[cb ^ 1][t] = ynext;
     __syncthreads();
     cb ^= 1;
@@ -568,8 +589,9 @@ __global__ __launch_bounds__(256) void k_wilson_lds(const cplx<R>* __restrict__ 
   uint4* out4 = reinterpret_cast<uint4*>(out);
 #pragma unroll
   for (int k = 0; k < CPS; ++k) {
-    const int c = t + k * T, q = c / CPS, e = c - q * CPS, s = q / nrhs, r = q - s * nrhs;
-    if (x0 + s < V) out4[((size_t)(x0 + s) * nrhs + r) * CPS + e] = s_rec[pos(q, e)];
+    const int c = t + k * T;
+    const WilsonChunk w = wilson_chunk<CPS, RS>(c, per_site, inv_per_site);
+    if (x0 + w.s < V) out4[(size_t)x0 * per_site + c] = s_rec[w.pos];
   }
 }
 
@@ -613,7 +635,8 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
   const bool live = x < V;
   const GammaTab G = gamma_table();
 
-  for (int j = t; j < 8 * S; j += T) {  // j = s * 8 + h: consecutive lanes, consecutive entries
+  const int hops = (mask & 0xffu) ? 8 * S : 0;  // Mdiag needs no neighbours
+  for (int j = t; j < hops; j += T) {  // j = s * 8 + h: consecutive lanes, consecutive entries
     const int s = j >> 3, h = j & 7;
     const int y = x0 + s < V ? nbr[(size_t)(x0 + s) * 8 + h] : 0;
     s_nb[h][s] = y;
@@ -797,7 +820,7 @@ __global__ __launch_bounds__(192) void k_wilson_row(const cplx<R>* __restrict__ 
   };
 
   i32x4 nb4 = {0, 0, 0, 0};
-  if (t < 2 * S && x0 + (t >> 1) < V)
+  if ((mask & 0xffu) && t < 2 * S && x0 + (t >> 1) < V)
     nb4 = reinterpret_cast<const i32x4*>(nbr)[(size_t)x0 * 2 + t];
   issue(8);
   cplx<R> dk[2][2][6];
