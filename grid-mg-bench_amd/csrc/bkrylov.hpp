@@ -43,6 +43,7 @@ struct BSolver {
   virtual ~BSolver() {}
   virtual BKrylovStats solve(BBlas& bl, BLinOp<R>& A, BPrec<R>* P, const cplx<R>* b, cplx<R>* x,
                              bool x_zero, double tol, int maxit) = 0;
+  virtual void set_iterate_only(bool) {}  // as Solver::set_iterate_only
 };
 
 template <typename R>
@@ -135,6 +136,8 @@ class BGmres : public BSolver<R> {
         cplx<double>* dh1 = d_h_;
         cplx<double>* dh2 = d_h_ + (size_t)(j + 2) * nr;
         cplx<R>* vnext = V_ + (size_t)(j + 1) * n;
+        // the cycle ends with this step: nothing reads the next basis vectors
+        const bool last = j + 1 == m || st.iters + 1 >= maxit;
         bdots_dev<R>(bl, V_, n, j + 1, w_, sh_, true, dh1);
         bfetch(bl, reinterpret_cast<const double*>(dh1), 2 * (j + 2) * nr);
         std::vector<double> hn(nr), sum1(nr, 0.0), wn2(nr);
@@ -150,14 +153,14 @@ class BGmres : public BSolver<R> {
           if (live[r] && wn2[r] - sum1[r] < eta_ * wn2[r]) reorth = true;
         }
         if (!reorth) {
-          bsubnorm_dev<R>(dh1, V_, n, j + 1, w_, vnext, sh_, s);
+          if (!last) bsubnorm_dev<R>(dh1, V_, n, j + 1, w_, vnext, sh_, s);
         } else {
           // w' = w - V h1, then h2 = V^H w' and |w'|^2 (one fused pass when j < 24)
           if (!bmultisub_dots_dev<R>(bl, dh1, V_, n, j + 1, w_, sh_, dh2)) {
             bmultisub_dev<R>(dh1, V_, n, j + 1, w_, sh_, s);
             bdots_dev<R>(bl, V_, n, j + 1, w_, sh_, true, dh2);
           }
-          bsubnorm_dev<R>(dh2, V_, n, j + 1, w_, vnext, sh_, s);
+          if (!last) bsubnorm_dev<R>(dh2, V_, n, j + 1, w_, vnext, sh_, s);
           bfetch(bl, reinterpret_cast<const double*>(dh2), 2 * (j + 2) * nr);
           bool redo = false;
           std::vector<double> sum2(nr, 0.0), wn2b(nr);
@@ -180,7 +183,7 @@ class BGmres : public BSolver<R> {
               hn[r] = std::sqrt(tmp[r]);
               scale[r] = hn[r] > 0.0 ? 1.0 / hn[r] : 0.0;
             }
-            bconvert<R, R>(bl, w_, vnext, sh_, scale.data());
+            if (!last) bconvert<R, R>(bl, w_, vnext, sh_, scale.data());
           }
         }
         ++st.iters;
@@ -230,6 +233,12 @@ class BGmres : public BSolver<R> {
         for (int i = 0; i < k; ++i) y[(size_t)i * nr + r] = {yy[i].real(), yy[i].imag()};
       }
       bmultiaxpy<R>(bl, y.data(), flexible_ ? Z_ : V_, n, j, x, sh_);
+      if (iterate_only_ && st.iters >= maxit) {
+        for (int r = 0; r < nr; ++r)
+          if (!st.converged[r] && bnorm[r] > 0.0)
+            st.rel_res[r] = std::abs(g[(size_t)r * (m + 1) + jr[r]]) / bnorm[r];
+        break;
+      }
       A.apply(x, w_, s);
       ++st.applies;
       vsub<R>(b, w_, r_, n, s);
@@ -242,6 +251,7 @@ class BGmres : public BSolver<R> {
   }
 
   const BShape& shape() const { return sh_; }
+  void set_iterate_only(bool on) override { iterate_only_ = on; }
 
   // re-orthogonalisation threshold eta, as Gmres::set_reorth_eta
   void set_reorth_eta(double eta) {
@@ -253,6 +263,7 @@ class BGmres : public BSolver<R> {
   BShape sh_;
   int m_;
   bool flexible_;
+  bool iterate_only_ = false;
   double eta_ = 0.5;
   cplx<R>* V_ = nullptr;
   cplx<R>* Z_ = nullptr;

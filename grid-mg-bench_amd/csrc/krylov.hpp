@@ -56,6 +56,10 @@ struct Solver {
   virtual ~Solver() {}
   virtual KrylovStats solve(Blas& bl, LinOp<R>& A, Prec<R>* P, const cplx<R>* b, cplx<R>* x,
                             bool x_zero, double tol, int maxit) = 0;
+  // The caller takes x alone and reads no final residual: a solver may then
+  // report its recurrence's estimate where it stops at maxit, instead of an
+  // operator application and three vector passes for the true one.  x is the same.
+  virtual void set_iterate_only(bool) {}
 };
 
 template <typename R>
@@ -132,6 +136,8 @@ class Gmres : public Solver<R> {
         cplx<double>* dh1 = d_h_;
         cplx<double>* dh2 = d_h_ + (j + 2);
         cplx<R>* vnext = V_ + (size_t)(j + 1) * n;
+        // the cycle ends with this step: nothing reads the next basis vector
+        const bool last = j + 1 == m_ || st.iters + 1 >= maxit;
         vmultidot_dev<R>(bl, V_, n, j + 1, w_, n, true, dh1);
         fetch(bl, reinterpret_cast<const double*>(dh1), 2 * (j + 2));
         double sum1 = 0.0;
@@ -143,7 +149,7 @@ class Gmres : public Solver<R> {
         double hn;
         if (wn2 - sum1 >= eta_ * wn2) {
           // one projection suffices: v = (w - V h1) / sqrt(|w|^2 - |h1|^2)
-          vsubnorm_dev<R>(dh1, V_, n, j + 1, w_, vnext, n, s);
+          if (!last) vsubnorm_dev<R>(dh1, V_, n, j + 1, w_, vnext, n, s);
           hn = std::sqrt(wn2 - sum1);
         } else {
           // w' = w - V h1, then h2 = V^H w' and |w'|^2 (one fused pass when j < 24)
@@ -151,7 +157,7 @@ class Gmres : public Solver<R> {
             vmultisub_dev<R>(dh1, V_, n, j + 1, w_, n, s);
             vmultidot_dev<R>(bl, V_, n, j + 1, w_, n, true, dh2);
           }
-          vsubnorm_dev<R>(dh2, V_, n, j + 1, w_, vnext, n, s);   // v = (w' - V h2) / hn
+          if (!last) vsubnorm_dev<R>(dh2, V_, n, j + 1, w_, vnext, n, s);  // v = (w' - V h2) / hn
           fetch(bl, reinterpret_cast<const double*>(dh2), 2 * (j + 2));
           double sum2 = 0.0;
           for (int i = 0; i <= j; ++i) {
@@ -166,7 +172,7 @@ class Gmres : public Solver<R> {
             // strong cancellation: form w'' = w' - V h2 and take its norm directly
             vmultisub_dev<R>(dh2, V_, n, j + 1, w_, n, s);
             hn = std::sqrt(vnorm2<R>(bl, w_, n));
-            if (hn > 0.0) vconvert<R, R>(w_, vnext, n, 1.0 / hn, s);
+            if (hn > 0.0 && !last) vconvert<R, R>(w_, vnext, n, 1.0 / hn, s);
           }
         }
         for (int i = 0; i <= j; ++i) H[(size_t)i * m_ + j] = C(h[i].re, h[i].im);
@@ -205,6 +211,10 @@ class Gmres : public Solver<R> {
       }
       for (int i = 0; i < j; ++i) y[i] = {yy[i].real(), yy[i].imag()};
       vmultiaxpy<R>(bl, y.data(), flexible_ ? Z_ : V_, n, j, x, n);
+      if (iterate_only_ && st.iters >= maxit) {
+        st.rel_res = std::abs(g[j]) / bnorm;
+        break;
+      }
       // true residual
       A.apply(x, w_, s);
       ++st.applies;
@@ -215,6 +225,7 @@ class Gmres : public Solver<R> {
   }
 
   size_t n() const { return n_; }
+  void set_iterate_only(bool on) override { iterate_only_ = on; }
   // Re-orthogonalisation threshold eta (default 1/2, the Daniel-Gragg-
   // Kaufman-Stewart test).  One classical projection leaves the new vector
   // orthogonal to the basis to about u / sqrt(eta) (u the unit roundoff) and
@@ -229,6 +240,7 @@ class Gmres : public Solver<R> {
   size_t n_;
   int m_;
   bool flexible_;
+  bool iterate_only_ = false;
   double eta_ = 0.5;
   cplx<R>* V_ = nullptr;
   cplx<R>* Z_ = nullptr;

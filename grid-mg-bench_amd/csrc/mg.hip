@@ -513,6 +513,9 @@ struct MG : MGBase {
         lv.smoother = make_solver<R>(p.coarsest_solver, lv.n, p.coarsest_restart,
                                      hier_reorth_eta<R>());
       }
+      // the cycles read no level solver's final residual
+      lv.smoother->set_iterate_only(true);
+      if (lv.wrapper) lv.wrapper->set_iterate_only(true);
       MGC_HIP(hipMalloc(&lv.t1, lv.n * sizeof(cplx<R>)));
       MGC_HIP(hipMalloc(&lv.t2, lv.n * sizeof(cplx<R>)));
       MGC_HIP(hipMalloc(&lv.t3, lv.n * sizeof(cplx<R>)));
@@ -755,6 +758,7 @@ struct MG : MGBase {
       } else {
         st->smoother = bsolver(p.coarsest_solver, p.coarsest_restart);
       }
+      st->smoother->set_iterate_only(true);  // the cycles read no final residual
       BL.push_back(std::move(st));
     }
     for (int l = 0; l + 2 < p.nlevels; ++l) {
@@ -765,6 +769,7 @@ struct MG : MGBase {
       } else {
         auto g = std::make_unique<BGmres<R>>(BL[l + 1]->op->sh, p.wrapper_restart, true);
         g->set_reorth_eta(hier_reorth_eta<R>());
+        g->set_iterate_only(true);
         BL[l]->wrapper = std::move(g);
       }
     }
