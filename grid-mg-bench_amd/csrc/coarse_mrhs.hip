@@ -67,7 +67,7 @@ __global__ void k_link_swizzle(const cplx<R>* __restrict__ links, int N,
   // out index: ((((x*9 + p)*NMT + mt)*NKC + kc)*64 + lane)
   using M = MK<KIND>;
   typedef typename M::T T;
-  const int NMT = mrhs_mtiles(N), NKC = 2 * NMT * 16 / M::KC;
+  const int NMT = mrhs_mtiles(N), NKC = mrhs_kchunks(N, M::KC);
   size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (; t < total; t += stride) {
@@ -290,13 +290,14 @@ static void prepare_mrhs(mgc_coarse_op* op, int mp, hipStream_t s) {
   const int N = op->N, V = op->V;
   MGC_CHECK(mrhs_supported(N), MGC_ERR_SHAPE,
             "multi-rhs stencil supports nbasis 8, 16, 24, ..., 64 (multiples of 8)");
-  const int NP = mrhs_mtiles(N) * 16;  // padded operand size
+  const int KC = mp == MGC_F32 ? 16 : 32;
+  // 16-byte fragments of the padded operand
+  const size_t total = (size_t)V * 9 * mrhs_mtiles(N) * mrhs_kchunks(N, KC) * 64;
   if (op->mrhs_links) {
     MGC_HIP(hipFree(op->mrhs_links));
     op->mrhs_links = nullptr;
   }
-  const size_t eb = mp == MGC_F32 ? 4 : 2;
-  MGC_HIP(hipMalloc(&op->mrhs_links, (size_t)V * 9 * NP * NP * 2 * eb));
+  MGC_HIP(hipMalloc(&op->mrhs_links, total * sizeof(uint4)));
   if (!op->mrhs_scales) MGC_HIP(hipMalloc(&op->mrhs_scales, (size_t)V * 9 * sizeof(float)));
   const int unit = mp == MGC_F32;
   if (op->prec == MGC_F64)
@@ -306,8 +307,6 @@ static void prepare_mrhs(mgc_coarse_op* op, int mp, hipStream_t s) {
     k_link_scale<float><<<V * 9, 256, 0, s>>>((const cplx<float>*)op->links, N, op->mrhs_scales,
                                               unit);
   MGC_LAUNCH_CHECK();
-  const int KC = mp == MGC_F32 ? 16 : 32;
-  const size_t total = (size_t)V * 9 * (NP / 16) * (2 * NP / KC) * 64;
   const unsigned g = grid_for(total, 256, 16384);
   uint4* o = (uint4*)op->mrhs_links;
 #define SWZ(KIND, R)                                                                        \

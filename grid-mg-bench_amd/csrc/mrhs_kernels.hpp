@@ -9,10 +9,12 @@
 // across rhs: sU = sF / Ls) and :806-820 (Mdag = G5C M G5C).
 //
 // nbasis N is any multiple of 8 up to 64.  The link operand is padded with
-// zero rows and columns to the next multiple of 16 (mrhs_mtiles), so a padded
-// K entry of B' (read from the next input column, or the zeros of a buffer
-// range check) always meets a zero link entry, and rows past N are never
-// stored.  N % 8 == 0 keeps each lane's chunk of KCL/2 complex entries on one
+// zero rows to the next multiple of 16 (mrhs_mtiles) and zero columns to whole
+// K chunks (mrhs_kchunks), so a padded K entry of B' (read from the next input
+// column, or the zeros of a buffer range check) always meets a zero link entry,
+// and rows past N are never stored.  Against K padded like the rows, FP32 at N =
+// 8, 24, 40, 56 moves and multiplies 1/2 to 7/8: 8^4, 12 rhs 16 -> 11, 60 -> 43
+// and 136 -> 117 us at N = 8, 24, 40.  N % 8 == 0 keeps each lane's chunk of KCL/2 complex entries on one
 // side of N/2, where the Mdag sign changes.
 #pragma once
 #include <type_traits>
@@ -21,8 +23,11 @@
 
 namespace mgc {
 
-// 16-row m-tiles of an nbasis-N operand (rows and K padded to 16 * tiles)
+// 16-row m-tiles of an nbasis-N operand (rows padded to 16 * tiles)
 __host__ __device__ constexpr int mrhs_mtiles(int N) { return (N + 15) / 16; }
+// its chunks of KC along K = 2 N (FP32, KC = 16: none is padding, where K padded
+// like the rows would carry and multiply one chunk of zeros at N = 8, 24, 40, 56)
+__host__ __device__ constexpr int mrhs_kchunks(int N, int KC) { return (2 * N + KC - 1) / KC; }
 // nbasis for which every kernel variant is built (the others run the
 // LDS-staged variants only)
 constexpr bool mrhs_all_variants(int N) { return N == 32 || N == 64; }
@@ -181,10 +186,10 @@ __device__ __forceinline__ void mrhs_lds_site(
   using M = MK<KIND>;
   typedef typename M::T T;
   constexpr int NMT = mrhs_mtiles(N);   // 16-row m-tiles, the last one zero-padded
-  constexpr int NKC = 2 * NMT * 16 / M::KC;
+  constexpr int NKC = mrhs_kchunks(N, M::KC);
   constexpr int THREADS = NMT * 64;
   constexpr int NSLOT = NKC * NT * 64;
-  constexpr int SPT = NSLOT / THREADS;  // staged slots per thread
+  constexpr int SPT = (NSLOT + THREADS - 1) / THREADS;  // staged slots per thread
   constexpr int NCOL = NT * 8;          // rhs columns covered by the tiles
   constexpr bool SCALED = KIND != MGC_F32;
   static_assert(NCOL <= THREADS, "one thread per column for the scale table");
@@ -268,6 +273,8 @@ __device__ __forceinline__ void mrhs_lds_site(
     if (q9 > 0) __syncthreads();  // previous point's MFMA readers are done with sB
 #pragma unroll
     for (int q = 0; q < SPT; ++q) {
+      // the last slots may be those of some wavefronts only
+      if (NSLOT % THREADS != 0 && w + q * NMT >= NKC * NT) continue;
       if constexpr (SCALED)
         sB[threadIdx.x + q * THREADS] =
             bprime_perm(b[q], ssel, smask0 ^ (slot_neg(q) ? 0x80008000u : 0u));
@@ -736,10 +743,10 @@ __global__ __launch_bounds__(mrhs_mtiles(N) * 64, (mrhs_persistent_min_waves<KIN
   using M = MK<KIND>;
   typedef typename M::T T;
   constexpr int NMT = mrhs_mtiles(N);
-  constexpr int NKC = 2 * NMT * 16 / M::KC;
+  constexpr int NKC = mrhs_kchunks(N, M::KC);
   constexpr int THREADS = NMT * 64;
   constexpr int NSLOT = NKC * NT * 64;
-  constexpr int SPT = NSLOT / THREADS;
+  constexpr int SPT = (NSLOT + THREADS - 1) / THREADS;
   constexpr int NCOL = NT * 8;
   constexpr int SITE_FRAGS = 9 * NMT * NKC * 64;  // uint4 fragments of one site's links
   constexpr bool SCALED = KIND != MGC_F32;
@@ -829,7 +836,8 @@ __global__ __launch_bounds__(mrhs_mtiles(N) * 64, (mrhs_persistent_min_waves<KIN
       __syncthreads();
 #pragma unroll
       for (int q = 0; q < SPT; ++q)
-        sB[threadIdx.x + q * THREADS] = bprime<KIND>(b[q], u, cdag && shi[q]);
+        if (NSLOT % THREADS == 0 || w + q * NMT < NKC * NT)
+          sB[threadIdx.x + q * THREADS] = bprime<KIND>(b[q], u, cdag && shi[q]);
       __syncthreads();
       // where the next step's operands come from: this site's next point, or
       // the next site's first point (the self point)
