@@ -258,6 +258,15 @@ __device__ __forceinline__ void wilson_diag_term(cplx<R>* acc, const cplx<R>* __
                        sp);
 }
 
+// ph x for a gamma phase ph, +-1 or +-i times a scale, known at compile time: its
+// zero part is left out here, since the compiler may not drop 0 * x (two
+// operations of three in the projections; the finite values are the same).
+template <typename R>
+__device__ __forceinline__ cplx<R> phase_mul(cplx<R> ph, cplx<R> x) {
+  if (ph.im == R(0)) return {ph.re * x.re, ph.re * x.im};
+  return {-ph.im * x.im, ph.im * x.re};
+}
+
 // Hopping term p with the rank-2 spin projector: for the upper spins s = 0, 1
 // (g_mu maps them to s' = col(s) in {2, 3}),
 //   h_s = psi_s - sg ph(s) psi_s',  (1 - sg g_mu) psi at s' = -sg ph(s') h_s,
@@ -278,7 +287,7 @@ __device__ __forceinline__ void wilson_hop_apply(cplx<R>* acc, const GammaTab& G
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       const cplx<R> a = sp(s * 3 + j), b = sp(cs * 3 + j);
-      const cplx<R> t = cmul(ph, b);
+      const cplx<R> t = phase_mul(ph, b);
       h[s][j] = {a.re - t.re, a.im - t.im};
     }
   }
@@ -302,7 +311,7 @@ __device__ __forceinline__ void wilson_hop_apply(cplx<R>* acc, const GammaTab& G
       const cplx<R> ph = {(R)(0.5 * sg * G.re[mu][cs]), (R)(0.5 * sg * G.im[mu][cs])};
       acc[s * 3 + i].re -= R(0.5) * chi.re;
       acc[s * 3 + i].im -= R(0.5) * chi.im;
-      const cplx<R> t = cmul(ph, chi);
+      const cplx<R> t = phase_mul(ph, chi);
       acc[cs * 3 + i].re += t.re;
       acc[cs * 3 + i].im += t.im;
     }
@@ -370,7 +379,7 @@ __device__ __forceinline__ void wilson_hop_apply_row(cplx<R>* acc, const GammaTa
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       const cplx<R> a = sp(s * 3 + j), b = sp(cs * 3 + j);
-      const cplx<R> t = cmul(ph, b);
+      const cplx<R> t = phase_mul(ph, b);
       h[s][j] = {a.re - t.re, a.im - t.im};
     }
   }
@@ -389,7 +398,7 @@ __device__ __forceinline__ void wilson_hop_apply_row(cplx<R>* acc, const GammaTa
     const cplx<R> ph = {(R)(0.5 * sg * G.re[mu][cs]), (R)(0.5 * sg * G.im[mu][cs])};
     acc[s].re -= R(0.5) * chi.re;
     acc[s].im -= R(0.5) * chi.im;
-    const cplx<R> t = cmul(ph, chi);
+    const cplx<R> t = phase_mul(ph, chi);
     acc[cs].re += t.re;
     acc[cs].im += t.im;
   }
@@ -457,12 +466,16 @@ struct WilsonChunk {
   int s, off, pos;
 };
 template <int CPS, int RS>
-__device__ __forceinline__ WilsonChunk wilson_chunk(int c, int per_site, float inv_per_site) {
+__device__ __forceinline__ int wilson_chunk_pos(int c) {  // q * RS + e of q = c / CPS, e = c % CPS
   static_assert((CPS == 6 || CPS == 12) && RS == CPS + 1, "record layout");
+  return c + (int)(__umul24(c, CPS == 6 ? 10923 : 5462) >> 16);
+}
+template <int CPS, int RS>
+__device__ __forceinline__ WilsonChunk wilson_chunk(int c, int per_site, float inv_per_site) {
   WilsonChunk w;
   w.s = (int)(((float)c + 0.5f) * inv_per_site);
   w.off = c - (int)__umul24(w.s, per_site);
-  w.pos = c + (int)(__umul24(c, CPS == 6 ? 10923 : 5462) >> 16);  // q * RS + e, q = c / CPS
+  w.pos = wilson_chunk_pos<CPS, RS>(c);
   return w;
 }
 // Cooperative copy of T records of CPS 16-byte chunks into LDS: chunk
@@ -712,7 +725,7 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
 #pragma unroll
     for (int k = 0; k < CPS; ++k) {
       const int c = t + k * T;
-      s_rec4[rec_pos<CPS, RS>(c / CPS, c % CPS)] = nrec[k];
+      s_rec4[wilson_chunk_pos<CPS, RS>(c)] = nrec[k];
     }
 #pragma unroll
     for (int m = 0; m < LPT; ++m)
@@ -742,7 +755,7 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
   for (int k = 0; k < CPS; ++k) {
     const int c = t + k * T, s = (int)(chunk[k] & 63);
     if (x0 + s < V)
-      out4[(size_t)x0 * (nrhs * CPS) + c] = s_rec[rec_pos<CPS, RS>(c / CPS, c % CPS)];
+      out4[(size_t)x0 * (nrhs * CPS) + c] = s_rec[wilson_chunk_pos<CPS, RS>(c)];
   }
 }
 
