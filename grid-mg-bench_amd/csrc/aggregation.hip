@@ -701,61 +701,65 @@ __device__ __forceinline__ void cq_load_T(double* sT, const cplx<double>* __rest
 // dst = src T for the CQ_CH staged rows (T upper triangular: output column
 // tile nt needs K steps 0 .. 4 nt + 3 only; the skipped terms are exact
 // zeros).  Wavefront w computes row tile w / (WAVES / 2) and two column
-// tiles chosen so that every wavefront runs the same number of steps.
+// tiles chosen so that every wavefront runs the same number of steps; the two
+// share each row operand they both need (LDS reads bound these products).
 template <int NP>
 __device__ __forceinline__ void cq_times_T(const double* src, const double* sT, double* dst) {
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int lk = l >> 4, t = lk & 1;
-  int mt, nts[2];
-  if (NP == 32) {
-    mt = w >> 1;
-    nts[0] = (w & 1) ? 1 : 0;
-    nts[1] = (w & 1) ? 2 : 3;
-  } else {
-    mt = w;
-    nts[0] = 0;
-    nts[1] = 1;
-  }
+  const int mt = NP == 32 ? w >> 1 : w;
+  const int nt0 = NP == 32 ? w & 1 : 0, nt1 = NP == 32 ? 3 - (w & 1) : 1;  // nt0 < nt1
   const int m = mt * 16 + (l & 15);
+  const int n0 = nt0 * 16 + (l & 15), n1 = nt1 * 16 + (l & 15);
+  const int u = l & 1;
+  const double bsign = (t == 1 && u == 0) ? -1.0 : 1.0;
+  const double* arow = src + m * CqShape<NP>::LDP + lk;
+  const double* b0 = sT + (lk >> 1) * CqShape<NP>::LDP + 2 * (n0 >> 1) + (t ^ u);
+  const double* b1 = sT + (lk >> 1) * CqShape<NP>::LDP + 2 * (n1 >> 1) + (t ^ u);
+  cq_dx4 acc0 = {0.0, 0.0, 0.0, 0.0}, acc1 = {0.0, 0.0, 0.0, 0.0};
+  constexpr int BS = 2 * CqShape<NP>::LDP;  // b operands of one step and the next
+  int kg = 0;
+  for (; kg <= nt0; ++kg)
 #pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const int nt = nts[q];
-    const int n = nt * 16 + (l & 15), cq = n >> 1, u = n & 1;
-    const double bsign = (t == 1 && u == 0) ? -1.0 : 1.0;
-    cq_dx4 acc = {0.0, 0.0, 0.0, 0.0};
-    const int ksteps = 4 * (nt + 1);
-    for (int ks = 0; ks < ksteps; ++ks) {
-      const double a = src[m * CqShape<NP>::LDP + 4 * ks + lk];
-      const int i = 2 * ks + (lk >> 1);
-      const double b = bsign * sT[i * CqShape<NP>::LDP + 2 * cq + (t ^ u)];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+    for (int ks = 4 * kg; ks < 4 * kg + 4; ++ks) {
+      const double a = arow[4 * ks];
+      acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bsign * b0[ks * BS], acc0, 0, 0, 0);
+      acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bsign * b1[ks * BS], acc1, 0, 0, 0);
     }
+  for (; kg <= nt1; ++kg)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) dst[(mt * 16 + 4 * r + lk) * CqShape<NP>::LDP + n] = acc[r];
+    for (int ks = 4 * kg; ks < 4 * kg + 4; ++ks)
+      acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(arow[4 * ks], bsign * b1[ks * BS], acc1, 0, 0, 0);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    dst[(mt * 16 + 4 * r + lk) * CqShape<NP>::LDP + n0] = acc0[r];
+    dst[(mt * 16 + 4 * r + lk) * CqShape<NP>::LDP + n1] = acc1[r];
   }
 }
 
 // acc += src^H src over the CQ_CH staged rows, for this wavefront's Gram tiles
 // (tiles wholly below the diagonal are skipped: the factorisation reads the
-// upper triangle only)
+// upper triangle only).  A wavefront's tiles lie in one tile row, so they share
+// the A operand.
 template <int NP>
 __device__ __forceinline__ void cq_gram_acc(const double* src, cq_dx4* acc) {
   typedef CqShape<NP> S;
+  static_assert(S::NTL % S::GTPW == 0, "a wavefront's tiles share the tile row");
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int lk = l >> 4, t = lk & 1;
+  const int lk = l >> 4, t = lk & 1, u = l & 1;
   const double asign = t ? -1.0 : 1.0;
+  const double bsign = (t == 1 && u == 0) ? -1.0 : 1.0;
+  const int mt = w * S::GTPW / S::NTL, nt0 = w * S::GTPW % S::NTL;
+  if (mt * 16 >= (nt0 + S::GTPW) * 8) return;  // every tile below the diagonal
+  const double* arow = src + (lk >> 1) * S::LDP + 2 * (mt * 16 + (l & 15)) + t;
+  const double* brow = src + (lk >> 1) * S::LDP + 2 * ((nt0 * 16 + (l & 15)) >> 1) + (t ^ u);
 #pragma unroll
-  for (int q = 0; q < S::GTPW; ++q) {
-    const int tile = w * S::GTPW + q, mt = tile / S::NTL, nt = tile % S::NTL;
-    if (mt * 16 >= (nt + 1) * 8) continue;  // every c > every c' of the tile
-    const int c = mt * 16 + (l & 15);
-    const int n = nt * 16 + (l & 15), cq = n >> 1, u = n & 1;
-    const double bsign = (t == 1 && u == 0) ? -1.0 : 1.0;
-#pragma unroll 4
-    for (int ks = 0; ks < CQ_CH / 2; ++ks) {
-      const int m = 2 * ks + (lk >> 1);
-      const double a = asign * src[m * S::LDP + 2 * c + t];
-      const double b = bsign * src[m * S::LDP + 2 * cq + (t ^ u)];
+  for (int ks = 0; ks < CQ_CH / 2; ++ks) {
+    const double a = asign * arow[2 * ks * S::LDP];
+#pragma unroll
+    for (int q = 0; q < S::GTPW; ++q) {
+      if (mt * 16 >= (nt0 + q + 1) * 8) continue;
+      const double b = bsign * brow[2 * ks * S::LDP + 16 * q];
       acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[q], 0, 0, 0);
     }
   }
