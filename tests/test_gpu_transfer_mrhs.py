@@ -34,6 +34,7 @@ SHAPES = [
     ((16, 16, 8, 8), (2, 2, 2, 2), 8, 12, 2),   # 1024 blocks, no split
     ((6, 3, 3, 3), (3, 3, 3, 3), 5, 12, 8),     # at most 8 columns and 8 rhs, 81 sites
     ((4, 4, 4, 4), (2, 2, 4, 4), 8, 12, 9),
+    ((16, 16, 8, 8), (4, 2, 2, 2), 56, 12, 5),  # eight wavefronts, the largest LDS of project
 ]
 
 
