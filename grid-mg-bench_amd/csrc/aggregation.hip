@@ -602,6 +602,7 @@ __device__ void cq_factor(cplx<double> (*sG)[NS], cplx<double> (*sX)[NS],
     for (int j = 0; j < nb; ++j) {
       const double gjj = sG[j][j].re;
       double d = gjj;
+#pragma unroll 8
       for (int i = 0; i < j; ++i) d -= sG[i][j].re * sG[i][j].re + sG[i][j].im * sG[i][j].im;
       const bool bad = !(d > CHOLQR_PIVOT_FLOOR * gjj) || !(gjj > 0.0);
       const double rjj = bad ? 1.0 : sqrt(d);
@@ -609,6 +610,7 @@ __device__ void cq_factor(cplx<double> (*sG)[NS], cplx<double> (*sX)[NS],
       // row j of R: R[j][k] = (G[j][k] - sum_{i<j} conj(R[i][j]) R[i][k]) / R[j][j]
       for (int k = j + 1 + t; k < nb; k += 64) {
         cplx<double> a = sG[j][k];
+#pragma unroll 8
         for (int i = 0; i < j; ++i) {
           const cplx<double> rij = sG[i][j], rik = sG[i][k];
           a.re -= rij.re * rik.re + rij.im * rik.im;
@@ -627,6 +629,7 @@ __device__ void cq_factor(cplx<double> (*sG)[NS], cplx<double> (*sX)[NS],
       sX[j][j] = {1.0 / sG[j][j].re, 0.0};
       for (int i = j - 1; i >= 0; --i) {
         cplx<double> a = {0.0, 0.0};
+#pragma unroll 4
         for (int k = i + 1; k <= j; ++k) cmac(a, sG[i][k], sX[k][j]);
         const double inv = 1.0 / sG[i][i].re;
         sX[i][j] = {-a.re * inv, -a.im * inv};
