@@ -68,6 +68,29 @@ struct ModWalk {
   }
 };
 
+// Sum of the 256 threads' values sm[t] that belong to rhs rr, t ascending, when
+// thread t holds the rhs ((off + t) % C) / dof: runs of dof threads every C.  A
+// thread visits its own rhs's runs only; testing every thread's rhs took 256
+// dependent LDS reads, most of the time of a reduction on a coarse level.
+__device__ __forceinline__ void rhs_block_sum(const double (*sm)[2], int off, int C, int dof,
+                                              int rr, double& sr, double& si) {
+  sr = si = 0.0;
+  if (dof == C) {  // one rhs
+    off = 0;
+    C = dof = 256;
+  }
+  int lo = rr * dof - off;
+  if (lo + dof <= 0) lo += C;
+  for (; lo < 256; lo += C) {
+    const int hi = min(lo + dof, 256);
+#pragma unroll 4
+    for (int t = max(lo, 0); t < hi; ++t) {
+      sr += sm[t][0];
+      si += sm[t][1];
+    }
+  }
+}
+
 // rows [BD_ROWS*y, ...): <V_j, w>_r for j < k, |w|^2_r for j == k
 template <typename R>
 __global__ __launch_bounds__(256) void k_bdot_part(const cplx<R>* __restrict__ V, size_t ldv,
@@ -76,12 +99,10 @@ __global__ __launch_bounds__(256) void k_bdot_part(const cplx<R>* __restrict__ V
                                                    int C, int dof, int nrhs,
                                                    double* __restrict__ part) {
   __shared__ double sm[BD_ROWS][256][2];
-  __shared__ int s_rt[256];  // the rhs of each thread's elements
   const int j0 = blockIdx.y * BD_ROWS;
   const int nj = min(BD_ROWS, rows - j0);
   const size_t T = (size_t)gridDim.x * blockDim.x;
   const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  s_rt[threadIdx.x] = (int)((g % C) / dof);
   double re[BD_ROWS], im[BD_ROWS];
 #pragma unroll
   for (int jj = 0; jj < BD_ROWS; ++jj) re[jj] = im[jj] = 0.0;
@@ -111,13 +132,8 @@ __global__ __launch_bounds__(256) void k_bdot_part(const cplx<R>* __restrict__ V
   // per-rhs sums of this block, threads in ascending order
   for (int q = threadIdx.x; q < nj * nrhs; q += blockDim.x) {
     const int jj = q / nrhs, rr = q % nrhs;
-    double sr = 0.0, si = 0.0;
-    for (int t = 0; t < (int)blockDim.x; ++t) {
-      if (s_rt[t] == rr) {
-        sr += sm[jj][t][0];
-        si += sm[jj][t][1];
-      }
-    }
+    double sr, si;
+    rhs_block_sum(sm[jj], (int)((size_t)blockIdx.x * 256 % C), C, dof, rr, sr, si);
     double* o = part + ((((size_t)(j0 + jj) * nrhs + rr) * gridDim.x) + blockIdx.x) * 2;
     o[0] = sr;
     o[1] = si;
@@ -132,13 +148,11 @@ __global__ __launch_bounds__(256) void k_bdot_part_f2(const cplx<float>* __restr
                                                       size_t n, int C, int dof, int nrhs,
                                                       double* __restrict__ part) {
   __shared__ double sm[BD_ROWS][256][2];
-  __shared__ int s_rt[256];  // the rhs of each thread's element pairs
   const int j0 = blockIdx.y * BD_ROWS;
   const int nj = min(BD_ROWS, rows - j0);
   const size_t T = (size_t)gridDim.x * blockDim.x;
   const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t n2 = n / 2;
-  s_rt[threadIdx.x] = (int)((2 * (g % (size_t)(C / 2))) / dof);
   double re[BD_ROWS], im[BD_ROWS];
 #pragma unroll
   for (int jj = 0; jj < BD_ROWS; ++jj) re[jj] = im[jj] = 0.0;
@@ -169,13 +183,8 @@ __global__ __launch_bounds__(256) void k_bdot_part_f2(const cplx<float>* __restr
   __syncthreads();
   for (int q = threadIdx.x; q < nj * nrhs; q += blockDim.x) {
     const int jj = q / nrhs, rr = q % nrhs;
-    double sr = 0.0, si = 0.0;
-    for (int t = 0; t < (int)blockDim.x; ++t) {
-      if (s_rt[t] == rr) {
-        sr += sm[jj][t][0];
-        si += sm[jj][t][1];
-      }
-    }
+    double sr, si;
+    rhs_block_sum(sm[jj], (int)((size_t)blockIdx.x * 256 % (C / 2)), C / 2, dof / 2, rr, sr, si);
     double* o = part + ((((size_t)(j0 + jj) * nrhs + rr) * gridDim.x) + blockIdx.x) * 2;
     o[0] = sr;
     o[1] = si;
@@ -212,10 +221,8 @@ __global__ __launch_bounds__(256) void k_bmsub_dot(const cplx<double>* __restric
   __shared__ __align__(16) unsigned char s_raw[SUM_BYTES > STAGE_BYTES ? SUM_BYTES : STAGE_BYTES];
   double(&sm)[BD_ROWS][256][2] = *reinterpret_cast<double(*)[BD_ROWS][256][2]>(s_raw);
   Slot(*s_v)[256] = reinterpret_cast<Slot(*)[256]>(s_raw);
-  __shared__ int s_rt[256];  // the rhs of each thread's first element
   const size_t T = (size_t)gridDim.x * blockDim.x;
   const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  s_rt[threadIdx.x] = PAIRED ? (int)((2 * (g % (size_t)(C / 2))) / dof) : (int)((g % C) / dof);
   double re[KT + 1], im[KT];
 #pragma unroll
   for (int j = 0; j <= KT; ++j) re[j] = 0.0;
@@ -313,13 +320,9 @@ __global__ __launch_bounds__(256) void k_bmsub_dot(const cplx<double>* __restric
       const int nj = min(BD_ROWS, rows - j0);
       for (int q = threadIdx.x; q < nj * nrhs; q += blockDim.x) {
         const int jj = q / nrhs, rr = q % nrhs;
-        double sr = 0.0, si = 0.0;
-        for (int t = 0; t < (int)blockDim.x; ++t) {
-          if (s_rt[t] == rr) {
-            sr += sm[jj][t][0];
-            si += sm[jj][t][1];
-          }
-        }
+        double sr, si;
+        const int ct = PAIRED ? C / 2 : C, dt = PAIRED ? dof / 2 : dof;  // in threads
+        rhs_block_sum(sm[jj], (int)((size_t)blockIdx.x * 256 % ct), ct, dt, rr, sr, si);
         double* o = part + ((((size_t)(j0 + jj) * nrhs + rr) * gridDim.x) + blockIdx.x) * 2;
         o[0] = sr;
         o[1] = si;
@@ -665,11 +668,9 @@ __global__ __launch_bounds__(256) void k_bbicg_xr_dots(
     cplx<R>* __restrict__ x, cplx<R>* __restrict__ r, size_t n, int C, int dof, int nrhs,
     double* __restrict__ part) {
   __shared__ double sm[2][256][2];
-  __shared__ int s_rt[256];
   const size_t T = (size_t)gridDim.x * blockDim.x;
   const size_t g = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int q = (int)((g % C) / dof);  // this thread's rhs, the same for all its elements
-  s_rt[threadIdx.x] = q;
   double rr = 0.0, hr = 0.0, hi = 0.0;
   if (c[2 * nrhs + q].re != 0.0) {
     const cplx<double> al = c[q], om = c[nrhs + q];
@@ -699,13 +700,8 @@ __global__ __launch_bounds__(256) void k_bbicg_xr_dots(
   // per-rhs sums of this block, threads in ascending order (as k_bdot_part)
   for (int o = threadIdx.x; o < 2 * nrhs; o += blockDim.x) {
     const int jj = o / nrhs, rq = o % nrhs;
-    double sr = 0.0, si2 = 0.0;
-    for (int k = 0; k < (int)blockDim.x; ++k) {
-      if (s_rt[k] == rq) {
-        sr += sm[jj][k][0];
-        si2 += sm[jj][k][1];
-      }
-    }
+    double sr, si2;
+    rhs_block_sum(sm[jj], (int)((size_t)blockIdx.x * 256 % C), C, dof, rq, sr, si2);
     double* out = part + ((((size_t)jj * nrhs + rq) * gridDim.x) + blockIdx.x) * 2;
     out[0] = sr;
     out[1] = si2;
