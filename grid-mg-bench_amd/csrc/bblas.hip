@@ -91,14 +91,17 @@ __device__ __forceinline__ void rhs_block_sum(const double (*sm)[2], int off, in
   }
 }
 
-// rows [BD_ROWS*y, ...): <V_j, w>_r for j < k, |w|^2_r for j == k
+// rows [BD_ROWS*y, ...): <V_j, w>_r for j < k, |w|^2_r for j == k.  LDS for the
+// block sums is sized to the rows: 32 KB for a norm would leave half the
+// wavefronts, and their loads in flight, out.
 template <typename R>
 __global__ __launch_bounds__(256) void k_bdot_part(const cplx<R>* __restrict__ V, size_t ldv,
                                                    int k, int rows,
                                                    const cplx<R>* __restrict__ w, size_t n,
                                                    int C, int dof, int nrhs,
                                                    double* __restrict__ part) {
-  __shared__ double sm[BD_ROWS][256][2];
+  extern __shared__ double smem_d[];
+  double(*sm)[256][2] = reinterpret_cast<double(*)[256][2]>(smem_d);  // [min(rows, BD_ROWS)]
   const int j0 = blockIdx.y * BD_ROWS;
   const int nj = min(BD_ROWS, rows - j0);
   const size_t T = (size_t)gridDim.x * blockDim.x;
@@ -124,10 +127,11 @@ __global__ __launch_bounds__(256) void k_bdot_part(const cplx<R>* __restrict__ V
     }
   }
 #pragma unroll
-  for (int jj = 0; jj < BD_ROWS; ++jj) {
-    sm[jj][threadIdx.x][0] = re[jj];
-    sm[jj][threadIdx.x][1] = im[jj];
-  }
+  for (int jj = 0; jj < BD_ROWS; ++jj)
+    if (jj < nj) {
+      sm[jj][threadIdx.x][0] = re[jj];
+      sm[jj][threadIdx.x][1] = im[jj];
+    }
   __syncthreads();
   // per-rhs sums of this block, threads in ascending order
   for (int q = threadIdx.x; q < nj * nrhs; q += blockDim.x) {
@@ -147,7 +151,8 @@ __global__ __launch_bounds__(256) void k_bdot_part_f2(const cplx<float>* __restr
                                                       const cplx<float>* __restrict__ w,
                                                       size_t n, int C, int dof, int nrhs,
                                                       double* __restrict__ part) {
-  __shared__ double sm[BD_ROWS][256][2];
+  extern __shared__ double smem_d[];
+  double(*sm)[256][2] = reinterpret_cast<double(*)[256][2]>(smem_d);  // [min(rows, BD_ROWS)]
   const int j0 = blockIdx.y * BD_ROWS;
   const int nj = min(BD_ROWS, rows - j0);
   const size_t T = (size_t)gridDim.x * blockDim.x;
@@ -176,10 +181,11 @@ __global__ __launch_bounds__(256) void k_bdot_part_f2(const cplx<float>* __restr
     }
   }
 #pragma unroll
-  for (int jj = 0; jj < BD_ROWS; ++jj) {
-    sm[jj][threadIdx.x][0] = re[jj];
-    sm[jj][threadIdx.x][1] = im[jj];
-  }
+  for (int jj = 0; jj < BD_ROWS; ++jj)
+    if (jj < nj) {
+      sm[jj][threadIdx.x][0] = re[jj];
+      sm[jj][threadIdx.x][1] = im[jj];
+    }
   __syncthreads();
   for (int q = threadIdx.x; q < nj * nrhs; q += blockDim.x) {
     const int jj = q / nrhs, rr = q % nrhs;
@@ -463,15 +469,16 @@ void bdots_dev(BBlas& b, const cplx<R>* V, size_t ldv, int k, const cplx<R>* w,
     b.part_cap = cap;
   }
   const dim3 grid(nblk, (rows + BD_ROWS - 1) / BD_ROWS);
+  const size_t sh_sum = (size_t)std::min(rows, BD_ROWS) * 256 * 2 * sizeof(double);
   if constexpr (std::is_same<R, float>::value) {
     if (pairs)
-      k_bdot_part_f2<<<grid, 256, 0, b.s>>>(V, ldv, k, rows, w, sh.n, sh.cols(), sh.dof,
+      k_bdot_part_f2<<<grid, 256, sh_sum, b.s>>>(V, ldv, k, rows, w, sh.n, sh.cols(), sh.dof,
                                             sh.nrhs, b.d_part);
     else
-      k_bdot_part<R><<<grid, 256, 0, b.s>>>(V, ldv, k, rows, w, sh.n, sh.cols(), sh.dof,
+      k_bdot_part<R><<<grid, 256, sh_sum, b.s>>>(V, ldv, k, rows, w, sh.n, sh.cols(), sh.dof,
                                             sh.nrhs, b.d_part);
   } else {
-    k_bdot_part<R><<<grid, 256, 0, b.s>>>(V, ldv, k, rows, w, sh.n, sh.cols(), sh.dof, sh.nrhs,
+    k_bdot_part<R><<<grid, 256, sh_sum, b.s>>>(V, ldv, k, rows, w, sh.n, sh.cols(), sh.dof, sh.nrhs,
                                           b.d_part);
   }
   MGC_LAUNCH_CHECK();
