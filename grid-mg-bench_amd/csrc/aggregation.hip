@@ -1004,15 +1004,16 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
                           s);
   } else {
     MGC_CHECK(promote_nb_ok(prec, nb), MGC_ERR_SHAPE, PROMOTE_NB_MSG);
-    auto lds = [&](int lpr) {
-      return ((size_t)rct * 2 * nb + (size_t)nb * (256 / lpr + 1)) * es;
+    auto lds = [&](int rhs, int lpr) {
+      return ((size_t)rhs * 2 * nb + (size_t)nb * (256 / lpr + 1)) * es;
     };
     // FP32 with nb <= 32: one lane per row, 256-row tiles (half the barriers
-    // per panel); otherwise two (or four) lanes per row
-    const int lpr = prec == MGC_F32 && nb <= 32 && lds(1) <= 65536 ? 1
-                    : lds(2) <= 65536                               ? 2
-                                                                    : 4;
-    const size_t sh = lds(lpr);
+    // per panel); otherwise two (or four) lanes per row.  The lanes of a row are
+    // its partial sums, so the choice goes by the tile of four rhs for one rhs too.
+    const int lpr = prec == MGC_F32 && nb <= 32 && lds(4, 1) <= 65536 ? 1
+                    : lds(4, 2) <= 65536                               ? 2
+                                                                       : 4;
+    const size_t sh = lds(rct, lpr);
     // register prefetch depth: entries per thread of one tile, rounded up to a power of 2
     const int need = (256 / lpr * nb + 255) / 256;
     const int tpt = need <= 2 ? 2 : need <= 4 ? 4 : need <= 8 ? 8 : need <= 16 ? 16 : 32;

@@ -206,8 +206,18 @@ __global__ __launch_bounds__(512) void k_project_mfma(
 // leaves through LDS, so that a site's record is written in whole lines: stored
 // from the product's registers, each lane's 16 bytes are a write request of
 // their own (75 million of them at the size above, 1.68 ms against 0.6 ms).
+// An element's 2 nb real products go to promote_sums chains, added in pairs at
+// the end: the rounding error grows with the square root of a chain's length,
+// and there are no fewer chains than the vector form has lanes for a row (two in
+// FP64, four from nb 30 up; in FP32 one, two from nb 31, four from nb 60).
+// Against one chain throughout that costs nothing to 10% of the time (FP64, nb
+// 48, 12 rhs, 18^4: 290 -> 313 us) and takes the error at nb 48 from 3.3e-16 to
+// 1.8e-16, in FP32 from 1.8e-7 to 1.3e-7.
 // ---------------------------------------------------------------------------
 constexpr int promote_ew(bool fast) { return fast ? 3 : 2; }
+constexpr int promote_sums(int kp, size_t real) {
+  return kp * real >= 32 ? 4 : kp * real >= 16 || real == 8 ? 2 : 1;
+}
 // LDS entries of one site: nr x EC elements and 16 bytes against bank conflicts
 template <typename R>
 __host__ __device__ constexpr int promote_pitch(int nr, int ec) {
@@ -268,13 +278,29 @@ __global__ __launch_bounds__(256) void k_promote_mfma(const cplx<R>* __restrict_
   };
   // products of one row and their way to LDS as element e of the tile
   auto product = [&](const cplx<R>(&u)[KR], int e) __attribute__((always_inline)) {
-    acc_t re = {0, 0, 0, 0}, im = {0, 0, 0, 0};
+    // NS chains, two at a time
+    constexpr int NS = promote_sums(KP, sizeof(R)), NC = NS < 2 ? 1 : 2, TG = KR * NC / NS;
+    static_assert(KR % TG == 0, "whole groups of steps");
+    acc_t re, im;
 #pragma unroll
-    for (int t = 0; t < KR; ++t) {
-      re = Mfma<R>::go(a[t].re, u[t].re, re);
-      im = Mfma<R>::go(a[t].re, u[t].im, im);
-      re = Mfma<R>::go(nai[t], u[t].im, re);
-      im = Mfma<R>::go(a[t].im, u[t].re, im);
+    for (int t0 = 0; t0 < KR; t0 += TG) {
+      acc_t sr[NC], si[NC];
+#pragma unroll
+      for (int q = 0; q < NC; ++q) sr[q] = si[q] = acc_t{0, 0, 0, 0};
+#pragma unroll
+      for (int t = t0; t < t0 + TG; ++t) {
+        acc_t &r = sr[t % NC], &i = si[t % NC];
+        r = Mfma<R>::go(a[t].re, u[t].re, r);
+        i = Mfma<R>::go(a[t].re, u[t].im, i);
+        r = Mfma<R>::go(nai[t], u[t].im, r);
+        i = Mfma<R>::go(a[t].im, u[t].re, i);
+      }
+      if (NC == 2) {
+        sr[0] += sr[NC - 1];
+        si[0] += si[NC - 1];
+      }
+      re = t0 ? re + sr[0] : sr[0];
+      im = t0 ? im + si[0] : si[0];
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
