@@ -206,17 +206,19 @@ __global__ __launch_bounds__(512) void k_project_mfma(
 // leaves through LDS, so that a site's record is written in whole lines: stored
 // from the product's registers, each lane's 16 bytes are a write request of
 // their own (75 million of them at the size above, 1.68 ms against 0.6 ms).
-// An element's 2 nb real products go to promote_sums chains, added in pairs at
-// the end: the rounding error grows with the square root of a chain's length,
-// and there are no fewer chains than the vector form has lanes for a row (two in
-// FP64, four from nb 30 up; in FP32 one, two from nb 31, four from nb 60).
+// An element's 2 nb real products go to promote_chains chains at a time, new ones
+// every promote_steps steps: the rounding error grows with the square root of a
+// chain's length, and no chain is longer than those of the vector form, whose lanes
+// for a row are two (FP64, four from nb 30 up) or one (FP32, two from nb 31, four
+// from nb 60).
 // Against one chain throughout that costs nothing to 10% of the time (FP64, nb
-// 48, 12 rhs, 18^4: 290 -> 313 us) and takes the error at nb 48 from 3.3e-16 to
+// 48, 12 rhs, 18^4: 290 -> 306 us) and takes the error at nb 48 from 3.3e-16 to
 // 1.8e-16, in FP32 from 1.8e-7 to 1.3e-7.
 // ---------------------------------------------------------------------------
 constexpr int promote_ew(bool fast) { return fast ? 3 : 2; }
-constexpr int promote_sums(int kp, size_t real) {
-  return kp * real >= 32 ? 4 : kp * real >= 16 || real == 8 ? 2 : 1;
+constexpr int promote_chains(int kp, size_t real) { return kp * real >= 16 || real == 8 ? 2 : 1; }
+constexpr int promote_steps(int kp, size_t real) {
+  return real == 4 ? 8 : kp <= 3 ? 2 * kp : 4;
 }
 // LDS entries of one site: nr x EC elements and 16 bytes against bank conflicts
 template <typename R>
@@ -278,9 +280,8 @@ __global__ __launch_bounds__(256) void k_promote_mfma(const cplx<R>* __restrict_
   };
   // products of one row and their way to LDS as element e of the tile
   auto product = [&](const cplx<R>(&u)[KR], int e) __attribute__((always_inline)) {
-    // NS chains, two at a time
-    constexpr int NS = promote_sums(KP, sizeof(R)), NC = NS < 2 ? 1 : 2, TG = KR * NC / NS;
-    static_assert(KR % TG == 0, "whole groups of steps");
+    // NC chains at a time, new ones every TG steps
+    constexpr int NC = promote_chains(KP, sizeof(R)), TG = promote_steps(KP, sizeof(R));
     acc_t re, im;
 #pragma unroll
     for (int t0 = 0; t0 < KR; t0 += TG) {
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(256) void k_promote_mfma(const cplx<R>* __restrict_
 #pragma unroll
       for (int q = 0; q < NC; ++q) sr[q] = si[q] = acc_t{0, 0, 0, 0};
 #pragma unroll
-      for (int t = t0; t < t0 + TG; ++t) {
+      for (int t = t0; t < (t0 + TG < KR ? t0 + TG : KR); ++t) {
         acc_t &r = sr[t % NC], &i = si[t % NC];
         r = Mfma<R>::go(a[t].re, u[t].re, r);
         i = Mfma<R>::go(a[t].re, u[t].im, i);

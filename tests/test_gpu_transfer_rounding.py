@@ -65,7 +65,7 @@ def promote_lanes(prec, nb):
 
 
 @pytest.mark.parametrize("nrhs", [1, 2, 5])
-@pytest.mark.parametrize("prec,nb", [(0, 8), (0, 16), (0, 29), (0, 30), (0, 31), (0, 48), (0, 56),
+@pytest.mark.parametrize("prec,nb", [(0, 8), (0, 16), (0, 29), (0, 30), (0, 31), (0, 40), (0, 48), (0, 56),
                                      (1, 16), (1, 30), (1, 31), (1, 32), (1, 48), (1, 60),
                                      (1, 64)])
 def test_promote_error(gpu, prec, nb, nrhs):
