@@ -951,8 +951,10 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
   if (project) {
     void* part = nullptr;
     if (S > 1) {
-      const size_t need =
-          (size_t)a->Vc * ((nrhs + 15) / 16) * S * std::min(16, nrhs) * 2 * nb * es;
+      // for whole groups of four rhs: a call that was made once leaves the
+      // workspace of every call of its group, which a HIP graph may then capture
+      const int rp = std::min(16, (nrhs + 3) / 4 * 4);
+      const size_t need = (size_t)a->Vc * ((nrhs + 15) / 16) * S * rp * 2 * nb * es;
       if (need > a->part_bytes) {
         if (a->part) MGC_HIP(hipFree(a->part));
         a->part = nullptr;

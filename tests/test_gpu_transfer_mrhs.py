@@ -8,6 +8,8 @@ fields at an address that is no multiple of 16 bytes.
 Tolerances as in test_gpu_aggregation.py: relative L2 1e-13 in FP64 and 2e-6 in
 FP32, where basis and inputs are rounded to 2^-24 and the sums are FP32.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -100,3 +102,45 @@ def test_masked_project_of_many_rhs(gpu, prec):
                 ref = oracle.project(fd, blk, nb, B, f[:, r].astype(np.complex128), kind=kind,
                                      point=point)
                 assert rel(ref, got[:, r]) < tol, (point, kind, r)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("first,then", [(1, 4), (2, 3), (5, 8), (13, 16)])
+def test_wider_projection_of_a_group_of_four_is_capturable(gpu, first, then, prec):
+    """One block, so that its panel is split and the partial sums take a workspace:
+    the one that a call of `first` rhs leaves serves `then` rhs under capture, where
+    nothing can be allocated.  Every replay gives the eager result."""
+    print(f"[case] capture first={first} then={then} prec={prec}", flush=True)
+    fd, nb = (4, 4, 4, 4), 8
+    Vf = int(np.prod(fd))
+    dt = gpu.complex_dtype(prec)
+    agg = gpu.Aggregation(fd, fd, nb)
+    agg.set_basis(gpu.DeviceBuffer.from_numpy(gauss(nb * Vf * 12, 851)))
+    df = gpu.DeviceBuffer.from_numpy(gauss(Vf * then * 12, 852).astype(dt))
+    shape = (then, 2 * nb)
+    want, got = (gpu.DeviceBuffer(then * 2 * nb * np.dtype(dt).itemsize) for _ in range(2))
+    gpu.synchronize()
+    hip, s = gpu.lib(), gpu.Stream()  # the HIP runtime is a dependency of the library
+    agg.project(df, want, prec, first, stream=s)
+    s.sync()
+    graph, ex = ctypes.c_void_p(), ctypes.c_void_p()
+    st = ctypes.c_void_p(s.handle)
+    assert hip.hipStreamBeginCapture(st, 1) == 0  # thread-local mode
+    try:
+        agg.project(df, got, prec, then, stream=s)
+    finally:
+        end = hip.hipStreamEndCapture(st, ctypes.byref(graph))
+    assert end == 0
+    assert hip.hipGraphInstantiate(ctypes.byref(ex), graph, None, None, ctypes.c_size_t(0)) == 0
+    try:
+        for _ in range(3):
+            got.zero()
+            gpu.synchronize()
+            assert hip.hipGraphLaunch(ex, st) == 0
+            s.sync()
+            agg.project(df, want, prec, then, stream=s)
+            s.sync()
+            assert np.array_equal(got.to_numpy(dt, shape), want.to_numpy(dt, shape))
+    finally:
+        hip.hipGraphExecDestroy(ex)
+        hip.hipGraphDestroy(graph)
