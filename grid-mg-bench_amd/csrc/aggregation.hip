@@ -128,16 +128,16 @@ const cplx<float>* agg_basis32(mgc_aggregation* a, hipStream_t s) {
 
 // ---------------------------------------------------------------------------
 // project: c(xc)(rhs)(k, i) = sum_{xb in mask, e in k} conj(U(xc,xb,e,i)) f(fine(xc,xb))(rhs)(e)
-// for one rhs (RCT = 1) or up to four (RCT = 4; wider calls: transfer_mfma.hip).
-// One workgroup per coarse site.  Thread
+// for one rhs (RCT = 1) or chunks of four (RCT = 4; the matrix form of several rhs:
+// transfer_mfma.hip).  One workgroup per (coarse site, chunk).  Thread
 // (i = t % nb, g = t / nb) walks rows q = g, g+G, ... of the block panel:
 // the nb threads of a group read one row's nb basis entries (contiguous) and
 // the G groups consecutive rows, so a wavefront streams the panel coalesced;
 // f(q) is a same-address broadcast load.  Group partial sums meet in LDS.
 // When the coarse lattice has few sites, blockIdx.z splits each panel into
 // gridDim.z row ranges of rows_per rows; the workgroups then write partial
-// sums to part[xc * gridDim.z + z][nrhs][2][nb], which k_project_reduce adds in a
-// fixed order.
+// sums to part[(xc * gridDim.y + y) * gridDim.z + z][min(4, nrhs)][2][nb], which
+// k_project_reduce adds in a fixed order.
 // With W = 2 (FP32, even nb) a thread takes the two adjacent basis columns
 // i = 2 i2, 2 i2 + 1 of each row in one 16-byte load, as the FP64 form reads
 // one column in 16 bytes; each column's sum keeps the row order q, q + G, ...
@@ -161,11 +161,13 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
                                                  const cplx<R>* __restrict__ f,
                                                  cplx<R>* __restrict__ c,
                                                  const int* __restrict__ blk_fine, int nb, int Vb,
-                                                 int Ef, int nr, Lat4 blk, int kind, int point,
+                                                 int Ef, int nrhs, Lat4 blk, int kind, int point,
                                                  int rows_per, cplx<R>* __restrict__ part) {
   extern __shared__ unsigned char smem_raw[];
   cplx<R>* s_red = reinterpret_cast<cplx<R>*>(smem_raw);  // [G][RCT][2][nb]
   const int xc = blockIdx.x;
+  const int r0 = blockIdx.y * RCT;
+  const int nr = min(RCT, nrhs - r0);
   const int tid = threadIdx.x;
   const int nw = nb / W;  // threads per row
   const int G = blockDim.x / nw;
@@ -196,7 +198,7 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
           const int xb = qq / Ef, e = qq - xb * Ef;
           lo[v] = e < half;
           project_row<R, W>(Ub + (size_t)qq * nb + i, uu[v]);
-          fp[v] = f + (size_t)bf[xb] * nr * Ef + e;
+          fp[v] = f + ((size_t)bf[xb] * nrhs + r0) * Ef + e;
         }
         cplx<R> xv[PU][RCT];
 #pragma unroll
@@ -221,7 +223,7 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
       const int k = e >= half;
       cplx<R> u[W];
       project_row<R, W>(Ub + (size_t)q * nb + i, u);
-      const cplx<R>* fr = f + (size_t)bf[xb] * nr * Ef + e;
+      const cplx<R>* fr = f + ((size_t)bf[xb] * nrhs + r0) * Ef + e;
 #pragma unroll
       for (int r = 0; r < RCT; ++r)
         if (r < nr) {
@@ -247,9 +249,10 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
     cplx<R> t = {R(0), R(0)};
     for (int gg = 0; gg < G; ++gg) t = cadd(t, s_red[(size_t)gg * RCT * 2 * nb + o]);
     if (gridDim.z == 1)
-      c[(size_t)xc * nr * 2 * nb + o] = t;
+      c[((size_t)xc * nrhs + r0) * 2 * nb + o] = t;
     else
-      part[((size_t)xc * gridDim.z + blockIdx.z) * nr * 2 * nb + o] = t;
+      part[(((size_t)xc * gridDim.y + blockIdx.y) * gridDim.z + blockIdx.z) * min(RCT, nrhs) * 2 *
+               nb + o] = t;
   }
 }
 
@@ -933,7 +936,10 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
   // 1.24, (16, 4), (24, 3), (32, 2) 0.73 to 1.04, more than four rhs at most
   // 0.83; in FP64, where the products weigh more, (20, 4) 0.98 to 1.18.
   const bool full_tiles = prec == MGC_F32 || 4 * nb >= 3 * ((nb + 15) / 16 * 16);
-  const bool matrix = nrhs > 4 || (nrhs * nb >= 64 && full_tiles);
+  // Project's sums are short enough for the vector form's rounding error (k_project_mfma)
+  // on blocks of eight Dirac sites or more.
+  const bool matrix = (nrhs > 4 || (nrhs * nb >= 64 && full_tiles)) &&
+                      (!project || (a->Vb >= 8 && rows >= 96));
   const int rct = nrhs == 1 ? 1 : 4;
   // split each panel over S workgroups when the coarse lattice alone gives
   // fewer than ~1024 workgroups (at least 64 rows per workgroup; a workgroup
@@ -946,7 +952,7 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
   }
   const int rows_per = (rows + S - 1) / S;
   S = (rows + rows_per - 1) / rows_per;
-  const dim3 grid(a->Vc, 1, S);
+  const dim3 grid(a->Vc, (nrhs + 3) / 4, S);
   const size_t es = prec == MGC_F64 ? sizeof(cplx<double>) : sizeof(cplx<float>);
   if (project) {
     void* part = nullptr;
@@ -977,7 +983,8 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
     if (rct == 1) PROJECT_T(R, 1, W, basis);                                                  \
     else PROJECT_T(R, 4, W, basis);                                                           \
     if (S > 1)                                                                                \
-      project_reduce<R>((const cplx<R>*)part, (cplx<R>*)out, a->Vc, 1, S, nrhs, nb, 4, s);    \
+      project_reduce<R>((const cplx<R>*)part, (cplx<R>*)out, a->Vc, (int)grid.y, S, nrhs, nb, \
+                        4, s);                                                                \
   } while (0)
     if (prec == MGC_F64) {
       if (matrix)

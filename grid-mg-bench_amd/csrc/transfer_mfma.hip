@@ -70,12 +70,20 @@ __device__ __forceinline__ void load_run(const cplx<R>* p, cplx<R>* o) {
 // wavefront takes four sites at a time, one per lane group (the K index of the
 // product), and EU elements of each: lane (g, j) loads the basis entries
 // MT j .. MT j + MT - 1 of its site's rows and the elements of rhs j.  The
-// sums of EU elements (2 * 4 * EU products) start from zero and are then added
-// to the running sums, which keeps the rounding of a 4^4 block's 3072-term
-// sums at that of two short ones.  The wavefronts' sums meet in LDS.
+// products of CH elements (2 * 4 * CH of them) start from zero and are then added to
+// the running sums; the wavefronts' sums meet in LDS.  The rounding error grows with
+// the square root of the additions in a row, 8 CH and the running sums' after them;
+// the vector form, with two stages over a block's rows, makes 2 sqrt(rows) at best.
+// CH = 2 keeps below that from eight Dirac sites a block up (agg_transfer asks for
+// them).  Where a workgroup has 64 sites or more, FP32 affords all six elements of a
+// chirality in one chain, with fewer registers and additions; ranges shorter than
+// that of a split panel take one element in FP64 (nb to 32, where registers allow).
+// Error in FP32, nb 32: at 2^4 blocks 8.8e-8 (vector form 1.02e-7, six in a chain
+// 1.31e-7), at 4^4 1.46e-7 (2.7e-7).  Two in a chain throughout, three elements a
+// step in FP32: up to 1.18 times the time (32^4, 4^4 blocks, nb 16, 12 rhs).
 // Sites past the range or outside the mask enter as zeros on both sides.
 // ---------------------------------------------------------------------------
-template <typename R, int MT, bool VEC, bool FAST>
+template <typename R, int MT, bool VEC, bool FAST, int CH>
 __global__ __launch_bounds__(512) void k_project_mfma(
     const cplx<R>* __restrict__ U, const cplx<R>* __restrict__ f, cplx<R>* __restrict__ c,
     const int* __restrict__ blk_fine, int nb, int Vb, int Ef_, int nrhs, Lat4 blk, int kind,
@@ -83,7 +91,7 @@ __global__ __launch_bounds__(512) void k_project_mfma(
   typedef typename Mfma<R>::acc_t acc_t;
   // elements per step: as many loads in flight as the registers allow
   constexpr bool wide = sizeof(R) == 8;
-  constexpr int EU = FAST ? (wide ? 3 : 6) : wide ? 2 : 4;
+  constexpr int EU = !FAST ? (wide ? 2 : 4) : !wide && (CH == 6 || MT == 1) ? 6 : 3;
   const int Ef = FAST ? 12 : Ef_;
   const int half = Ef / 2;
   extern __shared__ unsigned char smem_raw[];
@@ -129,34 +137,34 @@ __global__ __launch_bounds__(512) void k_project_mfma(
           if constexpr (!FAST) x[e] = fp[ee];
         }
         if constexpr (FAST) load_run<R, EU, true>(fp + half * k + eb, x);
-#pragma unroll
-        for (int e = 0; e < EU; ++e) {
-          const bool in = ok && (FAST || eb + e < half);
-          if (!in) {
-            x[e] = {R(0), R(0)};
-#pragma unroll
-            for (int m = 0; m < MT; ++m) u[e][m] = {R(0), R(0)};
-          }
-        }
-        acc_t acc[MT][2];
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = acc_t{0, 0, 0, 0};
         // conj(u) x: re = u.re x.re + u.im x.im, im = u.re x.im - u.im x.re
 #pragma unroll
-        for (int e = 0; e < EU; ++e) {
-          const R nx = -x[e].re;
+        for (int e0 = 0; e0 < EU; e0 += CH) {
+          acc_t acc[MT][2];
 #pragma unroll
-          for (int m = 0; m < MT; ++m) {
-            acc[m][0] = Mfma<R>::go(u[e][m].re, x[e].re, acc[m][0]);
-            acc[m][1] = Mfma<R>::go(u[e][m].re, x[e].im, acc[m][1]);
-            acc[m][0] = Mfma<R>::go(u[e][m].im, x[e].im, acc[m][0]);
-            acc[m][1] = Mfma<R>::go(u[e][m].im, nx, acc[m][1]);
+          for (int m = 0; m < MT; ++m) acc[m][0] = acc[m][1] = acc_t{0, 0, 0, 0};
+#pragma unroll
+          for (int e = e0; e < (e0 + CH < EU ? e0 + CH : EU); ++e) {
+            const bool in = ok && (FAST || eb + e < half);
+            if (!in) {
+              x[e] = {R(0), R(0)};
+#pragma unroll
+              for (int m = 0; m < MT; ++m) u[e][m] = {R(0), R(0)};
+            }
+            const R nx = -x[e].re;
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+              acc[m][0] = Mfma<R>::go(u[e][m].re, x[e].re, acc[m][0]);
+              acc[m][1] = Mfma<R>::go(u[e][m].re, x[e].im, acc[m][1]);
+              acc[m][0] = Mfma<R>::go(u[e][m].im, x[e].im, acc[m][0]);
+              acc[m][1] = Mfma<R>::go(u[e][m].im, nx, acc[m][1]);
+            }
           }
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) tot[k][m][t] += acc[m][t];
         }
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) tot[k][m][t] += acc[m][t];
       }
     }
   }
@@ -386,8 +394,14 @@ void project_launch(const mgc_aggregation* a, const cplx<R>* U, const cplx<R>* i
   int waves = (size_t)grid.x * grid.y * grid.z < 2048 ? 8 : 4;
   while (waves > 1 && 4 * (waves - 1) >= sites_per) waves /= 2;
   const size_t sh = (size_t)waves / 2 * MT * 2 * 64 * sizeof(typename Mfma<R>::acc_t);
-  k_project_mfma<R, MT, VEC, FAST><<<grid, 64 * waves, sh, s>>>(
-      U, in, out, a->blk_fine, a->nb, a->Vb, a->Ef, nrhs, a->blk, kind, point, sites_per, part);
+  auto k = k_project_mfma<R, MT, VEC, FAST, 2>;
+  if constexpr (FAST && sizeof(R) == 4) {
+    if (sites_per >= 64) k = k_project_mfma<R, MT, VEC, FAST, 6>;
+  } else if constexpr (FAST && MT <= 2) {
+    if (sites_per < 64 && grid.z > 1) k = k_project_mfma<R, MT, VEC, FAST, 1>;
+  }
+  k<<<grid, 64 * waves, sh, s>>>(U, in, out, a->blk_fine, a->nb, a->Vb, a->Ef, nrhs, a->blk, kind,
+                                 point, sites_per, part);
   MGC_LAUNCH_CHECK();
   if (grid.z > 1) project_reduce<R>(part, out, a->Vc, nchunk, (int)grid.z, nrhs, a->nb, TRC, s);
 }

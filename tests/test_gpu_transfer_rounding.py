@@ -65,9 +65,9 @@ def promote_lanes(prec, nb):
 
 
 @pytest.mark.parametrize("nrhs", [1, 2, 5])
-@pytest.mark.parametrize("prec,nb", [(0, 8), (0, 16), (0, 29), (0, 30), (0, 31), (0, 40), (0, 48), (0, 56),
-                                     (1, 16), (1, 30), (1, 31), (1, 32), (1, 48), (1, 60),
-                                     (1, 64)])
+@pytest.mark.parametrize("prec,nb", [(0, 8), (0, 16), (0, 29), (0, 30), (0, 31), (0, 40),
+                                     (0, 48), (0, 56), (1, 16), (1, 30), (1, 31), (1, 32),
+                                     (1, 48), (1, 60), (1, 64)])
 def test_promote_error(gpu, prec, nb, nrhs):
     print(f"[case] promote rounding nb={nb} nrhs={nrhs} prec={prec}", flush=True)
     fd, blk, Ef = (8, 4, 4, 4), (2, 2, 2, 2), 12
@@ -99,3 +99,74 @@ def test_promote_error(gpu, prec, nb, nrhs):
     err = rms(got, want)
     print(f"error {err:.3e}, {lanes} partial sums on the host {model:.3e}", flush=True)
     assert err <= SLACK * model
+
+
+def split(total, parts):
+    """[lo, hi) of equal ranges, the last one shorter."""
+    per = -(-total // parts)
+    return [(lo, min(total, lo + per)) for lo in range(0, total, per)]
+
+
+def in_order(terms):
+    acc = terms[0]
+    for t in terms[1:]:
+        acc = add(acc, t)
+    return acc
+
+
+# fine lattice, block, elements per site
+PROJECT = [((8, 8, 8, 4), (2, 1, 1, 1), 12), ((8, 8, 8, 2), (2, 2, 1, 1), 12),
+           ((8, 8, 4, 4), (2, 2, 2, 2), 12), ((6, 6, 6, 6), (3, 3, 3, 3), 12),
+           ((4, 4, 4, 2), (2, 2, 1, 1), 128),
+           ((4, 4, 4, 4), (2, 2, 2, 2), 64)]
+
+
+@pytest.mark.parametrize("nrhs", [2, 5])
+@pytest.mark.parametrize("prec,nb", [(0, 16), (0, 24), (0, 32), (0, 48), (1, 16), (1, 24),
+                                     (1, 32), (1, 48), (1, 64)])
+@pytest.mark.parametrize("fd,blk,Ef", PROJECT)
+def test_project_error(gpu, fd, blk, Ef, prec, nb, nrhs):
+    """Against a panel's rows dealt to 256 / nb groups (twice as many in FP32, which
+    takes two columns a thread), the rows of a group and then the groups added in
+    order, over as many row ranges as fill the chip (1024 / (blocks * chunks of four
+    rhs), 64 rows at least), and the ranges added by 256 / (8 nb) threads each."""
+    print(f"[case] project rounding fd={fd} blk={blk} Ef={Ef} nb={nb} nrhs={nrhs} prec={prec}",
+          flush=True)
+    Vf, Vc = int(np.prod(fd)), int(np.prod(oracle.coarse_dims(fd, blk)))
+    ct = gpu.complex_dtype(prec)
+    B = gauss(nb * Vf * Ef, 843).astype(ct).reshape(nb, Vf, Ef)
+    f = gauss(Vf * nrhs * Ef, 844).astype(ct).reshape(Vf, nrhs, Ef)
+    agg = gpu.Aggregation(fd, blk, nb, Ef)
+    agg.set_basis(gpu.DeviceBuffer.from_numpy(B.astype(np.complex128)))
+    oc = gpu.DeviceBuffer(Vc * nrhs * 2 * nb * np.dtype(ct).itemsize)
+    agg.project(gpu.DeviceBuffer.from_numpy(f), oc, prec, nrhs)
+    gpu.synchronize()
+    got = oc.to_numpy(ct, (Vc, nrhs, 2, nb))
+    U = block_rows(fd, blk, B.transpose(1, 0, 2))     # [block][row][nb]
+    F = block_rows(fd, blk, f)                        # [block][row][rhs]
+    rows = U.shape[1]
+    sel = slice(0, max(1, 60000 // (nrhs * 2 * nb)))  # blocks compared
+    U, F, got = U[sel], F[sel], got[sel]
+    wgs = Vc * -(-nrhs // 4)
+    S = max(1, min(-(-1024 // wgs), rows // 64)) if wgs < 1024 else 1
+    G = 256 // nb * (2 if prec == 1 else 1)
+    zg = max(1, 256 // (8 * nb))
+    err, model = np.zeros(2), np.zeros(2)
+    for k in range(2):
+        mine = np.arange(rows) % Ef // (Ef // 2) == k
+        want = np.einsum("bqi,bqr->bri", U[:, mine].conj().astype(np.clongdouble),
+                         F[:, mine].astype(np.clongdouble))
+        ranges = []
+        for lo, hi in split(rows, S):
+            groups = []
+            for g in range(G):
+                acc = (np.zeros(want.shape, REAL[prec]),) * 2
+                for q in range(lo + g, hi, G):
+                    if mine[q]:
+                        acc = cmac(prec, acc, F[:, q, :, None], U[:, q, None, :], conj_b=True)
+                groups.append(acc)
+            ranges.append(in_order(groups))
+        re, im = in_order([in_order(ranges[z::zg]) for z in range(min(zg, len(ranges)))])
+        err[k], model[k] = rms(got[:, :, k], want), rms(re + 1j * im, want)
+    print(f"error {err}, on the host {model}", flush=True)
+    assert np.hypot(*err) <= SLACK * np.hypot(*model)
