@@ -929,18 +929,6 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
             project ? "project: F64 or F32 vectors" : "promote: F64 or F32 vectors");
   const int nb = a->nb;
   const int rows = a->Vb * a->Ef;
-  // The matrix form reads the basis once per 16 rhs, the vector forms once per
-  // four, but its 16 x 16 tiles are mostly padding when both nb and nrhs are
-  // small.  Matrix over vector time at (nb, nrhs), project + promote over 16^3 x
-  // 32 and 18^4 with 3^4 blocks: (12, 2), (12, 3) 1.06 to 1.3, (20, 3) 0.91 to
-  // 1.24, (16, 4), (24, 3), (32, 2) 0.73 to 1.04, more than four rhs at most
-  // 0.83; in FP64, where the products weigh more, (20, 4) 0.98 to 1.18.
-  const bool full_tiles = prec == MGC_F32 || 4 * nb >= 3 * ((nb + 15) / 16 * 16);
-  // Project's sums are short enough for the vector form's rounding error (k_project_mfma)
-  // on blocks of eight Dirac sites or more.
-  const bool matrix = (nrhs > 4 || (nrhs * nb >= 64 && full_tiles)) &&
-                      (!project || (a->Vb >= 8 && rows >= 96));
-  const int rct = nrhs == 1 ? 1 : 4;
   // split each panel over S workgroups when the coarse lattice alone gives
   // fewer than ~1024 workgroups (at least 64 rows per workgroup; a workgroup
   // of four rhs counted, the split of several rhs needs no more than that)
@@ -952,6 +940,22 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
   }
   const int rows_per = (rows + S - 1) / S;
   S = (rows + rows_per - 1) / rows_per;
+  // The matrix form reads the basis once per 16 rhs, the vector forms once per
+  // four, but its 16 x 16 tiles are mostly padding when both nb and nrhs are
+  // small.  Matrix over vector time at (nb, nrhs), project + promote over 16^3 x
+  // 32 and 18^4 with 3^4 blocks: (12, 2), (12, 3) 1.06 to 1.3, (20, 3) 0.91 to
+  // 1.24, (16, 4), (24, 3), (32, 2) 0.73 to 1.04, more than four rhs at most
+  // 0.83; in FP64, where the products weigh more, (20, 4) 0.98 to 1.18.
+  const bool full_tiles = prec == MGC_F32 || 4 * nb >= 3 * ((nb + 15) / 16 * 16);
+  // Project's chains of additions are no longer than the vector form's
+  // (k_project_mfma) on blocks of eight Dirac sites or more, and in a split panel of
+  // longer records from 192 rows a workgroup up (FP64, nb 32, 64 elements: 64 rows 1.05
+  // times its error).
+  const bool short_chains = a->Vb >= 8 && rows >= 96 &&
+                            (S == 1 || a->Ef == 12 || rows_per >= 192);
+  const bool matrix =
+      (nrhs > 4 || (nrhs * nb >= 64 && full_tiles)) && (!project || short_chains);
+  const int rct = nrhs == 1 ? 1 : 4;
   const dim3 grid(a->Vc, (nrhs + 3) / 4, S);
   const size_t es = prec == MGC_F64 ? sizeof(cplx<double>) : sizeof(cplx<float>);
   if (project) {
