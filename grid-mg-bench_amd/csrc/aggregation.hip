@@ -13,6 +13,7 @@
 #include "aggregation.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 namespace mgc {
@@ -257,47 +258,67 @@ __global__ __launch_bounds__(256) void k_project(const cplx<R>* __restrict__ U,
 }
 
 // c(xc)(y*rc + r)(kn) = sum over the S row ranges of the partial sums, rp =
-// min(rc, nrhs) rhs a row of them.  One workgroup per (xc, y): thread (o, zg) sums z = zg, zg + ZG, ... for output
-// o, and the ZG group sums are added in order in LDS.
+// min(rc, nrhs) rhs a row of them.  One workgroup per (xc, y): thread (o, zg) sums
+// z = zg, zg + ZG, ... for output o in runs of four, the loads of two runs together,
+// and the ZG group sums are added in order in LDS.  A group has a run or more, which
+// keeps the chains of additions short, for the rounding error and the time alike (with
+// as many groups as a workgroup has room for, 128 of them for three ranges: 8^4, 2^4
+// blocks, nb 1, one rhs, 12.7 us, now 10.7).
+constexpr int RUN = 4, ZG_MAX = 8;
 template <typename R>
 __global__ __launch_bounds__(256) void k_project_reduce(const cplx<R>* __restrict__ part,
                                                         cplx<R>* __restrict__ c, int nchunk,
-                                                        int S, int nrhs, int nb, int rc, int rp) {
+                                                        int S, int nrhs, int nb, int rc, int rp,
+                                                        int ZG) {
   extern __shared__ unsigned char smem_raw[];
   cplx<R>* s_acc = reinterpret_cast<cplx<R>*>(smem_raw);  // [ZG][rp*2*nb]
   const int no = rp * 2 * nb;
   const size_t xy = blockIdx.x;
   const int y = (int)(xy % nchunk), xc = (int)(xy / nchunk);
-  if (no > (int)blockDim.x) {  // wide outputs: one thread per output, z in order
-    for (int oo = threadIdx.x; oo < no; oo += blockDim.x) {
-      cplx<R> t = {R(0), R(0)};
-      for (int z = 0; z < S; ++z) t = cadd(t, part[(xy * S + z) * no + oo]);
-      const int r = oo / (2 * nb), kn = oo - r * 2 * nb;
-      if (y * rc + r < nrhs) c[((size_t)xc * nrhs + y * rc + r) * 2 * nb + kn] = t;
+  auto sum = [&](int o, int z0) {
+    const cplx<R>* p = part + xy * S * no + o;
+    cplx<R> acc = {R(0), R(0)};
+    for (; z0 < S; z0 += 2 * RUN * ZG) {
+      cplx<R> v[2][RUN];
+#pragma unroll
+      for (int q = 0; q < 2 * RUN; ++q) {
+        const int z = z0 + q * ZG;
+        v[q / RUN][q % RUN] = z < S ? p[(size_t)z * no] : cplx<R>{R(0), R(0)};
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int q = 1; q < RUN; ++q) v[h][0] = cadd(v[h][0], v[h][q]);
+        acc = cadd(acc, v[h][0]);
+      }
     }
+    return acc;
+  };
+  auto store = [&](int o, cplx<R> t) {
+    const int r = o / (2 * nb), kn = o - r * 2 * nb;
+    if (y * rc + r < nrhs) c[((size_t)xc * nrhs + y * rc + r) * 2 * nb + kn] = t;
+  };
+  if (ZG == 1) {
+    for (int o = threadIdx.x; o < no; o += blockDim.x) store(o, sum(o, 0));
     return;
   }
-  const int ZG = (int)blockDim.x / no;
   const int o = threadIdx.x % no, zg = threadIdx.x / no;
-  cplx<R> acc = {R(0), R(0)};
-  if (zg < ZG)
-    for (int z = zg; z < S; z += ZG) acc = cadd(acc, part[(xy * S + z) * no + o]);
-  if (zg < ZG) s_acc[zg * no + o] = acc;
+  if (zg < ZG) s_acc[zg * no + o] = sum(o, zg);
   __syncthreads();
-  for (int oo = threadIdx.x; oo < no; oo += blockDim.x) {
-    cplx<R> t = {R(0), R(0)};
-    for (int g = 0; g < ZG; ++g) t = cadd(t, s_acc[g * no + oo]);
-    const int r = oo / (2 * nb), kn = oo - r * 2 * nb;
-    if (y * rc + r < nrhs) c[((size_t)xc * nrhs + y * rc + r) * 2 * nb + kn] = t;
+  if (zg == 0) {
+    cplx<R> t = s_acc[o];
+    for (int g = 1; g < ZG; ++g) t = cadd(t, s_acc[g * no + o]);
+    store(o, t);
   }
 }
 
 template <typename R>
 void project_reduce(const cplx<R>* part, cplx<R>* out, int Vc, int nchunk, int S, int nrhs, int nb,
                     int rc, hipStream_t s) {
-  // ZG * (rp*2*nb) <= 256 entries of LDS
-  k_project_reduce<R><<<Vc * nchunk, 256, 256 * sizeof(cplx<R>), s>>>(
-      part, out, nchunk, S, nrhs, nb, rc, std::min(rc, nrhs));
+  const int rp = std::min(rc, nrhs), no = rp * 2 * nb;
+  const int ZG = std::max(1, std::min({256 / no, ZG_MAX, (S + RUN - 1) / RUN}));
+  k_project_reduce<R><<<Vc * nchunk, 256, (size_t)ZG * no * sizeof(cplx<R>), s>>>(
+      part, out, nchunk, S, nrhs, nb, rc, rp, ZG);
   MGC_LAUNCH_CHECK();
 }
 

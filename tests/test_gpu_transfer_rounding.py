@@ -117,12 +117,12 @@ def in_order(terms):
 # fine lattice, block, elements per site
 PROJECT = [((8, 8, 8, 4), (2, 1, 1, 1), 12), ((8, 8, 8, 2), (2, 2, 1, 1), 12),
            ((8, 8, 4, 4), (2, 2, 2, 2), 12), ((6, 6, 6, 6), (3, 3, 3, 3), 12),
-           ((4, 4, 4, 2), (2, 2, 1, 1), 128),
+           ((8, 8, 8, 8), (4, 4, 4, 4), 12), ((4, 4, 4, 2), (2, 2, 1, 1), 128),
            ((4, 4, 4, 4), (2, 2, 2, 2), 64)]
 
 
-@pytest.mark.parametrize("nrhs", [2, 5])
-@pytest.mark.parametrize("prec,nb", [(0, 16), (0, 24), (0, 32), (0, 48), (1, 16), (1, 24),
+@pytest.mark.parametrize("nrhs", [1, 2, 5])
+@pytest.mark.parametrize("prec,nb", [(0, 8), (0, 16), (0, 24), (0, 32), (0, 48), (1, 16), (1, 24),
                                      (1, 32), (1, 48), (1, 64)])
 @pytest.mark.parametrize("fd,blk,Ef", PROJECT)
 def test_project_error(gpu, fd, blk, Ef, prec, nb, nrhs):
