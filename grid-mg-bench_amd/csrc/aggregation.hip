@@ -329,9 +329,9 @@ template void project_reduce<double>(const cplx<double>*, cplx<double>*, int, in
 
 // ---------------------------------------------------------------------------
 // promote: f(fine(xc,xb))(rhs)(e) = sum_i c(xc)(rhs)(chirality(e), i) U(xc,xb,e,i)
-// for one rhs (RCT = 1) or up to four (RCT = 4; wider calls: transfer_mfma.hip).
-// One workgroup per coarse site.  The block's basis panel (rows q = (xb, e), nb entries each, row-major) is streamed in
-// tiles of 256/LPR rows: each tile is read with contiguous loads
+// for one rhs (RCT = 1) or chunks of four (RCT = 4; the matrix form of several rhs:
+// transfer_mfma.hip).  One workgroup per (coarse site, chunk).  The block's basis panel
+// (rows q = (xb, e), nb entries each, row-major) is streamed in tiles of 256/LPR rows: each tile is read with contiguous loads
 // (consecutive threads take consecutive panel entries), stored transposed in
 // LDS ([i][row], one row of padding against bank conflicts), and each group of
 // LPR adjacent lanes then sums one row, nb/LPR entries each, joined by lane
@@ -342,17 +342,19 @@ __global__ __launch_bounds__(256) void k_promote(const cplx<R>* __restrict__ U,
                                                  const cplx<R>* __restrict__ c,
                                                  cplx<R>* __restrict__ f,
                                                  const int* __restrict__ blk_fine, int nb, int Vb,
-                                                 int Ef, int nr, int rows_per) {
+                                                 int Ef, int nrhs, int rows_per) {
   extern __shared__ unsigned char smem_raw[];
   cplx<R>* s_c = reinterpret_cast<cplx<R>*>(smem_raw);  // [RCT][2][nb]
   constexpr int PR = 256 / LPR;                         // rows per tile
   constexpr int LD = PR + 1;
   cplx<R>* s_u = s_c + RCT * 2 * nb;                    // [nb][LD]
   const int xc = blockIdx.x;
+  const int r0 = blockIdx.y * RCT;
+  const int nr = min(RCT, nrhs - r0);
   const int tid = threadIdx.x;
   const int half = Ef / 2;
   for (int o = tid; o < nr * 2 * nb; o += blockDim.x)
-    s_c[o] = c[(size_t)xc * nr * 2 * nb + o];
+    s_c[o] = c[((size_t)xc * nrhs + r0) * 2 * nb + o];
   const int rows = Vb * Ef;
   const cplx<R>* Ub = U + (size_t)xc * rows * nb;
   const int* bf = blk_fine + (size_t)xc * Vb;
@@ -427,7 +429,7 @@ __global__ __launch_bounds__(256) void k_promote(const cplx<R>* __restrict__ U,
       const int xb = q / Ef, e = q - xb * Ef;
 #pragma unroll
       for (int r = 0; r < RCT; ++r)
-        if (r < nr) f[((size_t)bf[xb] * nr + r) * Ef + e] = acc[r];
+        if (r < nr) f[((size_t)bf[xb] * nrhs + r0 + r) * Ef + e] = acc[r];
     }
   }
 }
@@ -961,21 +963,38 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
   }
   const int rows_per = (rows + S - 1) / S;
   S = (rows + rows_per - 1) / rows_per;
-  // The matrix form reads the basis once per 16 rhs, the vector forms once per
-  // four, but its 16 x 16 tiles are mostly padding when both nb and nrhs are
-  // small.  Matrix over vector time at (nb, nrhs), project + promote over 16^3 x
-  // 32 and 18^4 with 3^4 blocks: (12, 2), (12, 3) 1.06 to 1.3, (20, 3) 0.91 to
-  // 1.24, (16, 4), (24, 3), (32, 2) 0.73 to 1.04, more than four rhs at most
-  // 0.83; in FP64, where the products weigh more, (20, 4) 0.98 to 1.18.
-  const bool full_tiles = prec == MGC_F32 || 4 * nb >= 3 * ((nb + 15) / 16 * 16);
-  // Project's chains of additions are no longer than the vector form's
-  // (k_project_mfma) on blocks of eight Dirac sites or more, and in a split panel of
-  // longer records from 192 rows a workgroup up (FP64, nb 32, 64 elements: 64 rows 1.05
-  // times its error).
-  const bool short_chains = a->Vb >= 8 && rows >= 96 &&
-                            (S == 1 || a->Ef == 12 || rows_per >= 192);
-  const bool matrix =
-      (nrhs > 4 || (nrhs * nb >= 64 && full_tiles)) && (!project || short_chains);
+  // The matrix form (transfer_mfma.hip) reads the basis once per 16 rhs, the vector
+  // form once per four, but its 16 x 16 tiles are mostly padding when nb and nrhs are
+  // small.  Matrix over vector time on 16^3 x 32 (4^4 blocks), 18^4 (3^4), 16^4 (2^4)
+  // and 8^4 (both):
+  // - two to four rhs, project + promote, at (nb, nrhs): (12, 2), (12, 3) 1.06 to 1.3,
+  //   (20, 3) 0.91 to 1.24, (16, 4), (24, 3), (32, 2) 0.73 to 1.04; in FP64, where the
+  //   products weigh more, (20, 4) 0.98 to 1.18;
+  // - more rhs: nb 6 to 48 0.1 to 1.1 (one 1.36); nb 1 to 4 below;
+  const bool f64 = prec == MGC_F64;
+  const bool full_tiles = !f64 || 4 * nb >= 3 * ((nb + 15) / 16 * 16);
+  bool matrix = nrhs > 4 || (nrhs * nb >= 64 && full_tiles);
+  if (project) {
+    // - nb 1 to 4 in large blocks of a large lattice: FP64 0.97 to 2.2 (4^4), 1.04 to
+    //   1.6 (3^4, five to eight rhs; 0.77 to 0.96 with more), FP32 1.02 to 1.5 (4^4,
+    //   five to eight rhs; 0.6 to 1.0 with more); smaller ones 0.1 to 1.0;
+    const bool thin = nb <= 4 && S == 1 && rows >= (f64 && nrhs <= 8 ? 768 : 2048) &&
+                      (f64 || nrhs <= 8);
+    // - few rhs and small blocks in split panels: 8^4, 2^4 blocks, nb 16 to 48 FP64 1.08
+    //   to 1.4, FP32 two rhs 1.2, four 0.8 to 0.98.
+    const bool few = nrhs <= 4 && S > 1 && rows < 768 && (f64 || nrhs < 4);
+    // Project's chains of additions are no longer than the vector form's
+    // (k_project_mfma) on blocks of eight Dirac sites or more, and in a split panel of
+    // longer records from 192 rows a workgroup up (FP64, nb 32, 64 elements: 64 rows
+    // 1.05 times its error).
+    const bool short_chains =
+        a->Vb >= 8 && rows >= 96 && (S == 1 || a->Ef == 12 || rows_per >= 192);
+    matrix = matrix && short_chains && !thin && !few;
+  } else {
+    // - nb 1 to 4: 3^4 blocks (sites no multiple of the 16 columns) 0.9 to 1.9 at any
+    //   nrhs, others 0.8 to 1.26 up to eight rhs and 0.7 to 1.3 with more.
+    matrix = matrix && !(nb <= 4 && (nrhs <= 8 || a->Vb % 16 != 0));
+  }
   const int rct = nrhs == 1 ? 1 : 4;
   const dim3 grid(a->Vc, (nrhs + 3) / 4, S);
   const size_t es = prec == MGC_F64 ? sizeof(cplx<double>) : sizeof(cplx<float>);

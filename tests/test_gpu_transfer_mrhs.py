@@ -1,5 +1,5 @@
-"""Project and promote of several right-hand sides (the matrix-core form) at the
-edges of its tiles: basis widths around multiples of 16 and 4 (odd ones among
+"""Project and promote of several right-hand sides (the matrix-core form, and the
+vector form in chunks of four where the dispatch keeps it) at the edges of its tiles: basis widths around multiples of 16 and 4 (odd ones among
 them), 16-rhs column tiles with remainders, blocks whose site count is no
 multiple of a wavefront's four or sixteen sites, fields of a coarse level
 (element counts other than 12), masks, panels split over workgroups, and FP32
@@ -37,6 +37,14 @@ SHAPES = [
     ((6, 3, 3, 3), (3, 3, 3, 3), 5, 12, 8),     # at most 8 columns and 8 rhs, 81 sites
     ((4, 4, 4, 4), (2, 2, 4, 4), 8, 12, 9),
     ((16, 16, 8, 8), (4, 2, 2, 2), 56, 12, 5),  # eight wavefronts, the largest LDS of project
+    # narrow bases, both sides of the rules that keep the vector form, in chunks of four
+    ((4, 4, 4, 4), (2, 2, 2, 2), 4, 12, 9),
+    ((6, 3, 3, 3), (3, 3, 3, 3), 3, 12, 9),
+    ((3, 3, 3, 6), (3, 3, 3, 3), 4, 12, 17),
+    ((12, 12, 12, 24), (3, 3, 3, 3), 2, 12, 7),   # 512 blocks, two chunks: no split
+    ((12, 12, 12, 24), (3, 3, 3, 3), 4, 12, 10),
+    ((16, 16, 16, 16), (4, 4, 4, 4), 1, 12, 13),
+    ((8, 4, 4, 4), (2, 2, 2, 1), 32, 12, 3),      # split small blocks, few rhs
 ]
 
 
