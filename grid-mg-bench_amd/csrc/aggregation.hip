@@ -33,21 +33,23 @@ __global__ __launch_bounds__(IB_THREADS) void k_import_basis(
     const int* __restrict__ blk_fine, cplx<double>* __restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
   cplx<double>* s_t = reinterpret_cast<cplx<double>*>(smem_raw);  // [IB_ROWS][nb + 1]
-  const size_t q0 = (size_t)blockIdx.x * IB_ROWS;
-  const int n = (int)(rows - q0 < (size_t)IB_ROWS ? rows - q0 : (size_t)IB_ROWS);
   const int r = threadIdx.x % IB_ROWS;
-  if (r < n) {
-    const size_t q = q0 + r;
-    const int e = (int)(q % Ef);
-    const cplx<double>* p = src + (size_t)blk_fine[q / Ef] * Ef + e;
-    const size_t vec = (size_t)Vf * Ef;
+  const size_t vec = (size_t)Vf * Ef;
+  for (size_t q0 = (size_t)blockIdx.x * IB_ROWS; q0 < rows; q0 += (size_t)gridDim.x * IB_ROWS) {
+    const int n = (int)(rows - q0 < (size_t)IB_ROWS ? rows - q0 : (size_t)IB_ROWS);
+    if (r < n) {
+      const size_t q = q0 + r;
+      const int e = (int)(q % Ef);
+      const cplx<double>* p = src + (size_t)blk_fine[q / Ef] * Ef + e;
 #pragma unroll 4
-    for (int i = threadIdx.x / IB_ROWS; i < nb; i += IB_THREADS / IB_ROWS)
-      s_t[r * (nb + 1) + i] = p[i * vec];
+      for (int i = threadIdx.x / IB_ROWS; i < nb; i += IB_THREADS / IB_ROWS)
+        s_t[r * (nb + 1) + i] = p[i * vec];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < n * nb; t += IB_THREADS)
+      dst[q0 * nb + t] = s_t[t + t / nb];  // row t / nb of pitch nb + 1
+    __syncthreads();
   }
-  __syncthreads();
-  for (int t = threadIdx.x; t < n * nb; t += IB_THREADS)
-    dst[q0 * nb + t] = s_t[t + t / nb];  // row t / nb of pitch nb + 1
 }
 
 __global__ void k_export_basis(const cplx<double>* __restrict__ src, int nb, int Vf, int Ef,
@@ -1197,7 +1199,7 @@ int mgc_aggregation_set_basis(mgc_aggregation* a, const void* basis_f64, void* s
     MGC_CHECK(a && basis_f64, MGC_ERR_ARG, "null argument");
     const size_t rows = (size_t)a->Vf * a->Ef;
     hipStream_t s = as_stream(stream);
-    k_import_basis<<<(unsigned)((rows + IB_ROWS - 1) / IB_ROWS), IB_THREADS,
+    k_import_basis<<<tile_grid((rows + IB_ROWS - 1) / IB_ROWS), IB_THREADS,
                      (size_t)IB_ROWS * (a->nb + 1) * sizeof(cplx<double>), s>>>(
         (const cplx<double>*)basis_f64, a->nb, a->Vf, a->Ef, rows, a->blk_fine, a->basis64);
     MGC_LAUNCH_CHECK();

@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256) void k_import_links_tiled(
   }
 }
 
-// The converse, one workgroup per 32 x 32 tile of a (site, point) matrix: the
+// The converse, a workgroup at a time per 32 x 32 tile of a (site, point) matrix: the
 // links are read along their columns (r fastest) and the external layouts
 // written along their rows (c fastest), 512-byte runs on both sides through
 // LDS.  A copy bound by HBM: 8^4, N = 64, FP64 (4.8 GB) 0.90 ms, 2.75 ms with
@@ -235,25 +235,26 @@ constexpr int EXT = 32;
 template <typename R>
 __global__ __launch_bounds__(256) void k_export_links(const cplx<R>* __restrict__ links,
                                                       int layout, int V, int N, int nt,
+                                                      size_t tiles,
                                                       cplx<double>* __restrict__ dst) {
   __shared__ cplx<R> sA[EXT][EXT + 1];  // [c][r]
-  int b = blockIdx.x;
-  const int tc = b % nt;
-  b /= nt;
-  const int tr = b % nt;
-  b /= nt;
-  const int p = b % 9, x = b / 9;
   const int i = threadIdx.x % EXT, j0 = threadIdx.x / EXT;
-  const cplx<R>* src = links + ((size_t)x * 9 + p) * N * N;  // [c][r]
-  for (int j = j0; j < EXT; j += 256 / EXT) {
-    const int c = tc * EXT + j, r = tr * EXT + i;
-    if (c < N && r < N) sA[j][i] = src[c * N + r];
-  }
-  __syncthreads();
-  for (int j = j0; j < EXT; j += 256 / EXT) {
-    const int r = tr * EXT + j, c = tc * EXT + i;
-    if (c < N && r < N)
-      dst[ext_link_index(layout, V, N, p, x, r, c)] = {(double)sA[i][j].re, (double)sA[i][j].im};
+  for (size_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const size_t m = tile / (nt * nt);  // matrix (x, p)
+    const int rem = (int)(tile - m * (nt * nt)), tr = rem / nt, tc = rem - tr * nt;
+    const int x = (int)(m / 9), p = (int)(m - (size_t)x * 9);
+    const cplx<R>* src = links + m * N * N;  // [c][r]
+    for (int j = j0; j < EXT; j += 256 / EXT) {
+      const int c = tc * EXT + j, r = tr * EXT + i;
+      if (c < N && r < N) sA[j][i] = src[c * N + r];
+    }
+    __syncthreads();
+    for (int j = j0; j < EXT; j += 256 / EXT) {
+      const int r = tr * EXT + j, c = tc * EXT + i;
+      if (c < N && r < N)
+        dst[ext_link_index(layout, V, N, p, x, r, c)] = {(double)sA[i][j].re, (double)sA[i][j].im};
+    }
+    __syncthreads();
   }
 }
 
@@ -720,13 +721,14 @@ int mgc_coarse_op_get_links(const mgc_coarse_op* op, int layout, void* links_f64
               "unknown link layout");
     hipStream_t s = as_stream(stream);
     const int nt = (op->N + EXT - 1) / EXT;
-    const unsigned g = (unsigned)((size_t)op->V * 9 * nt * nt);
+    const size_t tiles = (size_t)op->V * 9 * nt * nt;
+    const unsigned g = tile_grid(tiles);
     if (op->prec == MGC_F64)
       k_export_links<double><<<g, 256, 0, s>>>((const cplx<double>*)op->links, layout, op->V,
-                                               op->N, nt, (cplx<double>*)links_f64);
+                                               op->N, nt, tiles, (cplx<double>*)links_f64);
     else if (op->prec == MGC_F32)
       k_export_links<float><<<g, 256, 0, s>>>((const cplx<float>*)op->links, layout, op->V,
-                                              op->N, nt, (cplx<double>*)links_f64);
+                                              op->N, nt, tiles, (cplx<double>*)links_f64);
     else
       throw Error(MGC_ERR_PRECISION, "no single-rhs links in a half-precision operator");
     MGC_LAUNCH_CHECK();

@@ -622,39 +622,39 @@ __global__ __launch_bounds__(256, 3) void k_coarsen_mfma(
 }
 
 // A_want(x) = sigma o adj(A_have(x + disp_want * mu)), FLAT layout, in place:
-// one workgroup per 32 x 32 tile of a link, transposed through LDS so that both
-// sides run along rows.  Bound by HBM (8^4, N = 64: 2.1 GB).
+// a workgroup at a time per 32 x 32 tile of a link, transposed through LDS so that
+// both sides run along rows.  Bound by HBM (8^4, N = 64: 2.1 GB).
 constexpr int RT = 32;
 __global__ __launch_bounds__(256) void k_reconstruct(cplx<double>* __restrict__ links, Lat4 lat,
-                                                     int N, int nt, int disp_have,
+                                                     int N, int nt, size_t tiles, int disp_have,
                                                      const int* __restrict__ nbr) {
   __shared__ cplx<double> sA[RT][RT + 1];
   const int V = lat.volume(), nb = N / 2;
-  int b = blockIdx.x;
-  const int tc = b % nt;
-  b /= nt;
-  const int tr = b % nt;
-  b /= nt;
-  const int x = b % V, mu = b / V;
-  const int ph = disp_have > 0 ? mu : mu + 4;  // point we have
-  const int pw = disp_have > 0 ? mu + 4 : mu;  // point we want
-  // neighbour in direction disp_want = -disp_have: the want-point's own neighbour
-  const int y = nbr[(size_t)x * 8 + pw];
-  const cplx<double>* have = links + ((size_t)ph * V + y) * N * N;
-  cplx<double>* want = links + ((size_t)pw * V + x) * N * N;
   const int i = threadIdx.x % RT, j0 = threadIdx.x / RT;
-  for (int j = j0; j < RT; j += 256 / RT) {  // element (c, r) of the link we have
-    const int c = tc * RT + j, r = tr * RT + i;
-    if (c < N && r < N) sA[j][i] = have[(size_t)c * N + r];
-  }
-  __syncthreads();
-  for (int j = j0; j < RT; j += 256 / RT) {
-    const int r = tr * RT + j, c = tc * RT + i;
-    if (r >= N || c >= N) continue;
-    cplx<double> a = sA[i][j];
-    a.im = -a.im;
-    if ((r / nb + c / nb) & 1) { a.re = -a.re; a.im = -a.im; }
-    want[(size_t)r * N + c] = a;
+  for (size_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const size_t m = tile / (nt * nt);  // link (mu, x)
+    const int rem = (int)(tile - m * (nt * nt)), tr = rem / nt, tc = rem - tr * nt;
+    const int mu = (int)(m / V), x = (int)(m - (size_t)mu * V);
+    const int ph = disp_have > 0 ? mu : mu + 4;  // point we have
+    const int pw = disp_have > 0 ? mu + 4 : mu;  // point we want
+    // neighbour in direction disp_want = -disp_have: the want-point's own neighbour
+    const int y = nbr[(size_t)x * 8 + pw];
+    const cplx<double>* have = links + ((size_t)ph * V + y) * N * N;
+    cplx<double>* want = links + ((size_t)pw * V + x) * N * N;
+    for (int j = j0; j < RT; j += 256 / RT) {  // element (c, r) of the link we have
+      const int c = tc * RT + j, r = tr * RT + i;
+      if (c < N && r < N) sA[j][i] = have[(size_t)c * N + r];
+    }
+    __syncthreads();
+    for (int j = j0; j < RT; j += 256 / RT) {
+      const int r = tr * RT + j, c = tc * RT + i;
+      if (r >= N || c >= N) continue;
+      cplx<double> a = sA[i][j];
+      a.im = -a.im;
+      if ((r / nb + c / nb) & 1) { a.re = -a.re; a.im = -a.im; }
+      want[(size_t)r * N + c] = a;
+    }
+    __syncthreads();
   }
 }
 
@@ -726,8 +726,9 @@ static void launch_coarsen(const mgc_aggregation* agg, const mgc_fine_op* fop, c
 static void reconstruct(cplx<double>* links, const mgc_coarse_op* cop, int disp_have,
                         hipStream_t s) {
   const int nt = (cop->N + RT - 1) / RT;
-  k_reconstruct<<<(unsigned)((size_t)4 * cop->V * nt * nt), 256, 0, s>>>(
-      links, cop->lat, cop->N, nt, disp_have, cop->nbr_full);
+  const size_t tiles = (size_t)4 * cop->V * nt * nt;
+  k_reconstruct<<<tile_grid(tiles), 256, 0, s>>>(links, cop->lat, cop->N, nt, tiles, disp_have,
+                                                 cop->nbr_full);
   MGC_LAUNCH_CHECK();
 }
 

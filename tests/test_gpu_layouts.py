@@ -57,3 +57,54 @@ def test_basis_round_trip(gpu, fd, blk, nb, Ef):
     ref = oracle.project_ef(fd, blk, nb, Ef, B, f)
     got = oc.to_numpy(np.complex128, (Vc, 2 * nb))
     assert np.linalg.norm(got - ref) < 1e-13 * np.linalg.norm(ref)
+
+
+def part(gpu, buf, first, shape):
+    """Elements [first, ...) of a complex128 buffer."""
+    out = np.empty(shape, np.complex128)
+    gpu.call("mgc_memcpy_d2h", out.ctypes.data, buf.ptr + first * 16, out.nbytes, None)
+    gpu.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("N,dims,prec", [(50, (8, 8, 8, 4), 1), (34, (26, 26, 26, 27), 1)])
+def test_links_round_trip_of_many_tiles(gpu, N, dims, prec):
+    """More tiles than one launch has workgroups, and more than one launch may have work
+    items (132 GB in all): the first, last and some sites between."""
+    print(f"[case] many tiles N={N} dims={dims}", flush=True)
+    V = int(np.prod(dims))
+    buf = gpu.DeviceBuffer(9 * V * N * N * 16)
+    gpu.random_gaussian(buf, 9 * V * N * N, gpu.F64, 5, 861)
+    at = [(p, x) for p in (0, 4, 8) for x in (0, 1, V // 3, V // 2 + 1, V - 2)]
+    want = [part(gpu, buf, (p * V + x) * N * N, (2, N, N)) for p, x in at]
+    op = gpu.CoarseOp(dims, N, prec)
+    op.set_links(buf, gpu.LAYOUT_FLAT, invert=False)
+    buf.zero()
+    op.get_links(buf, gpu.LAYOUT_FLAT)
+    gpu.synchronize()
+    for (p, x), w in zip(at, want):
+        got = part(gpu, buf, (p * V + x) * N * N, (2, N, N))
+        assert np.array_equal(got, w.astype(gpu.complex_dtype(prec)).astype(np.complex128)), (p, x)
+    buf.close()
+    op.close()
+
+
+@pytest.mark.parametrize("dims,blk,nb,Ef", [((32, 16, 32, 32), (2, 2, 2, 1), 4, 12),
+                                            ((64, 64, 32, 33), (2, 4, 1, 3), 1, 256)])
+def test_basis_round_trip_of_many_tiles(gpu, dims, blk, nb, Ef):
+    """As above (18 GB a copy): the import against the export."""
+    print(f"[case] many tiles basis dims={dims} blk={blk} nb={nb} Ef={Ef}", flush=True)
+    V = int(np.prod(dims))
+    src, back = gpu.DeviceBuffer(nb * V * Ef * 16), gpu.DeviceBuffer(nb * V * Ef * 16)
+    gpu.random_gaussian(src, nb * V * Ef, gpu.F64, 5, 862)
+    agg = gpu.Aggregation(dims, blk, nb, Ef)
+    agg.set_basis(src)
+    agg.get_basis(back)
+    gpu.synchronize()
+    for i in (0, nb - 1):
+        for x in (0, 1, V // 3, V // 2 + 1, V - 2):
+            first = (i * V + x) * Ef
+            assert np.array_equal(part(gpu, back, first, (2, Ef)), part(gpu, src, first, (2, Ef)))
+    src.close()
+    back.close()
+    agg.close()
