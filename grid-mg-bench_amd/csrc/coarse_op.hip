@@ -193,7 +193,7 @@ __global__ void k_import_links(const cplx<double>* __restrict__ src, int layout,
   }
 }
 
-// The same import, one workgroup per (site, point) matrix through LDS: the
+// The same import, a workgroup at a time per (site, point) matrix through LDS: the
 // source is read along its rows (c fastest, contiguous in both layouts) and
 // the column-major destination written along its columns (r fastest), so
 // both sides are coalesced.  For N <= 64.
@@ -202,27 +202,30 @@ __global__ __launch_bounds__(256) void k_import_links_tiled(
     const cplx<double>* __restrict__ src, int layout, int V, int N, cplx<R>* __restrict__ links,
     cplx<R>* __restrict__ self_dag, cplx<double>* __restrict__ self_rm) {
   __shared__ cplx<double> sA[64][65];
-  const int x = blockIdx.x / 9, p = blockIdx.x - x * 9;
   const int t = threadIdx.x;
-  for (int idx = t; idx < N * N; idx += 256) {
-    const int r = idx / N, c = idx - r * N;
-    sA[r][c] = src[ext_link_index(layout, V, N, p, x, r, c)];
-  }
-  __syncthreads();
-  cplx<R>* dst = links + ((size_t)x * 9 + p) * N * N;  // [c][r]
-  for (int idx = t; idx < N * N; idx += 256) {
-    const int c = idx / N, r = idx - c * N;
-    const cplx<double> a = sA[r][c];
-    dst[idx] = {(R)a.re, (R)a.im};
-  }
-  if (p == 8) {
-    // adj(A8) column-major: element (row r, col c) = conj(A8(c, r)), at [c][r]
+  for (size_t m = blockIdx.x; m < (size_t)V * 9; m += gridDim.x) {
+    const int x = (int)(m / 9), p = (int)(m - (size_t)x * 9);
+    for (int idx = t; idx < N * N; idx += 256) {
+      const int r = idx / N, c = idx - r * N;
+      sA[r][c] = src[ext_link_index(layout, V, N, p, x, r, c)];
+    }
+    __syncthreads();
+    cplx<R>* dst = links + m * N * N;  // [c][r]
     for (int idx = t; idx < N * N; idx += 256) {
       const int c = idx / N, r = idx - c * N;
-      const cplx<double> b = sA[c][r];
-      self_dag[(size_t)x * N * N + idx] = {(R)b.re, (R)(-b.im)};
-      self_rm[(size_t)x * N * N + idx] = sA[c][r];  // row-major: idx = row c, column r
+      const cplx<double> a = sA[r][c];
+      dst[idx] = {(R)a.re, (R)a.im};
     }
+    if (p == 8) {
+      // adj(A8) column-major: element (row r, col c) = conj(A8(c, r)), at [c][r]
+      for (int idx = t; idx < N * N; idx += 256) {
+        const int c = idx / N, r = idx - c * N;
+        const cplx<double> b = sA[c][r];
+        self_dag[(size_t)x * N * N + idx] = {(R)b.re, (R)(-b.im)};
+        self_rm[(size_t)x * N * N + idx] = sA[c][r];  // row-major: idx = row c, column r
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -662,14 +665,14 @@ int mgc_coarse_op_set_links(mgc_coarse_op* op, int layout, const void* links_f64
     cplx<double>* rm = nullptr;
     MGC_HIP(hipMalloc(&rm, (size_t)V * N * N * sizeof(cplx<double>)));
     const size_t total = (size_t)V * 9 * N * N;
-    const unsigned g = grid_for(total, 256, 16384);
+    const unsigned g = grid_for(total, 256, 16384), gt = tile_grid((size_t)V * 9);
     const auto* lf = (const cplx<double>*)links_f64;
     if (op->prec == MGC_F64 && N <= 64)
-      k_import_links_tiled<double><<<V * 9, 256, 0, s>>>(lf, layout, V, N, (cplx<double>*)op->links,
-                                                         (cplx<double>*)op->self_dag, rm);
+      k_import_links_tiled<double><<<gt, 256, 0, s>>>(lf, layout, V, N, (cplx<double>*)op->links,
+                                                      (cplx<double>*)op->self_dag, rm);
     else if (op->prec == MGC_F32 && N <= 64)
-      k_import_links_tiled<float><<<V * 9, 256, 0, s>>>(lf, layout, V, N, (cplx<float>*)op->links,
-                                                        (cplx<float>*)op->self_dag, rm);
+      k_import_links_tiled<float><<<gt, 256, 0, s>>>(lf, layout, V, N, (cplx<float>*)op->links,
+                                                     (cplx<float>*)op->self_dag, rm);
     else if (op->prec == MGC_F64)
       k_import_links<double><<<g, 256, 0, s>>>(lf, layout, V, N, (cplx<double>*)op->links,
                                                (cplx<double>*)op->self_dag, rm);

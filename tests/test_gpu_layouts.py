@@ -67,7 +67,8 @@ def part(gpu, buf, first, shape):
     return out
 
 
-@pytest.mark.parametrize("N,dims,prec", [(50, (8, 8, 8, 4), 1), (34, (26, 26, 26, 27), 1)])
+@pytest.mark.parametrize("N,dims,prec", [(50, (8, 8, 8, 4), 1), (34, (26, 26, 26, 27), 1),
+                                         (2, (38, 37, 36, 37), 0), (2, (38, 37, 36, 37), 1)])
 def test_links_round_trip_of_many_tiles(gpu, N, dims, prec):
     """More tiles than one launch has workgroups, and more than one launch may have work
     items (132 GB in all): the first, last and some sites between."""
