@@ -658,6 +658,39 @@ __global__ __launch_bounds__(256) void k_reconstruct(cplx<double>* __restrict__ 
   }
 }
 
+// The same for whole_matrices, `mats` links at a time (as k_export_links_whole).
+__global__ __launch_bounds__(256) void k_reconstruct_whole(cplx<double>* __restrict__ links,
+                                                           Lat4 lat, int N, int mats,
+                                                           int disp_have,
+                                                           const int* __restrict__ nbr) {
+  extern __shared__ unsigned char smem_raw[];
+  cplx<double>* sA = reinterpret_cast<cplx<double>*>(smem_raw);  // [link][r][c], rows N + 1 apart
+  const unsigned V = lat.volume(), nb = N / 2, N2 = N * N;
+  for (size_t m0 = (size_t)blockIdx.x * mats; m0 < (size_t)4 * V; m0 += (size_t)gridDim.x * mats) {
+    const size_t left = (size_t)4 * V - m0;
+    const unsigned n = (unsigned)(left < (size_t)mats ? left : mats) * N2;
+    for (unsigned i = threadIdx.x; i < n; i += 256) {
+      const unsigned q = i / N2;
+      const size_t m = m0 + q;  // (mu, x)
+      const unsigned mu = (unsigned)(m / V), x = (unsigned)(m - (size_t)mu * V);
+      const unsigned ph = disp_have > 0 ? mu : mu + 4, pw = disp_have > 0 ? mu + 4 : mu;
+      const unsigned y = nbr[(size_t)x * 8 + pw];
+      sA[i + i / N] = links[((size_t)ph * V + y) * N2 + (i - q * N2)];
+    }
+    __syncthreads();
+    for (unsigned i = threadIdx.x; i < n; i += 256) {
+      const unsigned q = i / N2, rc = i - q * N2, r = rc / N, c = rc - r * N;
+      const size_t m = m0 + q;
+      const unsigned mu = (unsigned)(m / V), x = (unsigned)(m - (size_t)mu * V);
+      cplx<double> a = sA[(q * N + c) * (N + 1) + r];
+      a.im = -a.im;
+      if ((r / nb + c / nb) & 1) { a.re = -a.re; a.im = -a.im; }
+      links[((size_t)(disp_have > 0 ? mu + 4 : mu) * V + x) * N2 + rc] = a;
+    }
+    __syncthreads();
+  }
+}
+
 template <int NB, int TC>
 static void launch_coarsen_t(const mgc_aggregation* agg, const mgc_fine_op* fop, const int* plist,
                              int np, cplx<double>* links, hipStream_t s) {
@@ -725,10 +758,19 @@ static void launch_coarsen(const mgc_aggregation* agg, const mgc_fine_op* fop, c
 
 static void reconstruct(cplx<double>* links, const mgc_coarse_op* cop, int disp_have,
                         hipStream_t s) {
-  const int nt = (cop->N + RT - 1) / RT;
-  const size_t tiles = (size_t)4 * cop->V * nt * nt;
-  k_reconstruct<<<tile_grid(tiles), 256, 0, s>>>(links, cop->lat, cop->N, nt, tiles, disp_have,
-                                                 cop->nbr_full);
+  const int N = cop->N;
+  const size_t mats = (size_t)4 * cop->V;
+  if (whole_matrices(N)) {
+    const int per = std::max(1, 1024 / (N * N));
+    k_reconstruct_whole<<<tile_grid((mats + per - 1) / per), 256,
+                          (size_t)per * N * (N + 1) * sizeof(cplx<double>), s>>>(
+        links, cop->lat, N, per, disp_have, cop->nbr_full);
+  } else {
+    const int nt = (N + RT - 1) / RT;
+    const size_t tiles = mats * nt * nt;
+    k_reconstruct<<<tile_grid(tiles), 256, 0, s>>>(links, cop->lat, N, nt, tiles, disp_have,
+                                                   cop->nbr_full);
+  }
   MGC_LAUNCH_CHECK();
 }
 

@@ -162,6 +162,6 @@ inline unsigned grid_for(size_t n, unsigned block, unsigned cap = 65535u * 8u) {
 
 // number of workgroups for a kernel that loops over tiles (HIP refuses launches of
 // 2^32 work items or more)
-inline unsigned tile_grid(size_t tiles) { return grid_for(tiles, 1, 65536); }
+inline unsigned tile_grid(size_t tiles) { return grid_for(tiles, 1, 1u << 22); }
 
 }  // namespace mgc

@@ -1,6 +1,6 @@
-"""Exact round trips through the tiled layout conversions: links (32 x 32 tiles,
-both external layouts) and basis (48 panel rows a tile), at sizes with partial
-tiles.  Values are moved, not computed: equality bit for bit (FP32 operators:
+"""Exact round trips through the tiled layout conversions: links (whole matrices up
+to N = 48, 32 x 32 tiles above; both external layouts) and basis (48 panel rows a
+tile), at sizes with partial tiles.  Values are moved, not computed: equality bit for bit (FP32 operators:
 equality with the rounded input)."""
 import numpy as np
 import pytest
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", [0, 1])
-@pytest.mark.parametrize("N", [2, 30, 32, 34, 64, 66])
+@pytest.mark.parametrize("N", [2, 6, 14, 30, 32, 34, 48, 50, 64, 66])
 def test_links_round_trip(gpu, N, prec):
     print(f"[case] links N={N} prec={prec}", flush=True)
     dims = (2, 1, 3, 2)
@@ -32,6 +32,24 @@ def test_links_round_trip(gpu, N, prec):
     got = out.to_numpy(np.complex128, (9, V, 2, 2, N // 2, N // 2))
     split = want.reshape(9, V, 2, N // 2, 2, N // 2).transpose(0, 1, 2, 4, 3, 5)
     assert np.array_equal(got, split)
+
+
+@pytest.mark.parametrize("disp_have", [1, -1])
+@pytest.mark.parametrize("N", [2, 12, 32, 34, 48, 50])
+def test_reconstructed_links(gpu, N, disp_have):
+    """Links are conjugated and moved: equality bit for bit."""
+    print(f"[case] reconstruct N={N} disp_have={disp_have}", flush=True)
+    dims = (2, 5, 3, 2)
+    V = int(np.prod(dims))
+    links = rand_links(dims, N)
+    op = gpu.CoarseOp(dims, N, gpu.F64)
+    op.set_links(gpu.DeviceBuffer.from_numpy(links), gpu.LAYOUT_FLAT, invert=False)
+    gpu.construct_remaining_links(op, disp_have)
+    out = gpu.DeviceBuffer(links.nbytes)
+    op.get_links(out, gpu.LAYOUT_FLAT)
+    gpu.synchronize()
+    want = oracle.construct_remaining_links(dims, N, links, disp_have).reshape(9, V, N, N)
+    assert np.array_equal(out.to_numpy(np.complex128, want.shape), want)
 
 
 @pytest.mark.parametrize("fd,blk,nb,Ef", [((2, 3, 1, 1), (1, 3, 1, 1), 1, 2),
@@ -67,11 +85,11 @@ def part(gpu, buf, first, shape):
     return out
 
 
-@pytest.mark.parametrize("N,dims,prec", [(50, (8, 8, 8, 4), 1), (34, (26, 26, 26, 27), 1),
+@pytest.mark.parametrize("N,dims,prec", [(34, (26, 26, 26, 27), 1), (50, (18, 18, 18, 20), 1),
                                          (2, (38, 37, 36, 37), 0), (2, (38, 37, 36, 37), 1)])
 def test_links_round_trip_of_many_tiles(gpu, N, dims, prec):
-    """More tiles than one launch has workgroups, and more than one launch may have work
-    items (132 GB in all): the first, last and some sites between."""
+    """More tiles than one launch has workgroups, or more than it may have work items
+    (132 GB and 70 GB in all for the first two): the first, last and some sites between."""
     print(f"[case] many tiles N={N} dims={dims}", flush=True)
     V = int(np.prod(dims))
     buf = gpu.DeviceBuffer(9 * V * N * N * 16)
