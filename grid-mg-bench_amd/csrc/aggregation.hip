@@ -22,27 +22,30 @@ namespace mgc {
 // layout conversion
 // ---------------------------------------------------------------------------
 // Basis vectors [i][site][e] to panels [row][i] (row = (block, block site, e)),
-// IB_ROWS panel rows a workgroup through LDS: a thread keeps its row and reads
-// it of every IB_ROWS-th vector (runs of whole sites, 768 bytes where a block
-// is four sites wide), and the tile leaves as one contiguous run.  A copy bound
+// ROWS panel rows at a time through LDS: a thread keeps its row and reads
+// it of every (IB_THREADS / ROWS)-th vector (runs of whole sites, 768 bytes where a
+// block is four sites wide), and the tile leaves as one contiguous run.  A copy bound
 // by HBM: 32^4, nb 32 (12.9 GB) 2.46 ms (5.2 TB/s), 4.3 ms with the panel order
-// on both sides.
-constexpr int IB_ROWS = 48, IB_THREADS = 192;
+// on both sides.  Bases of up to four vectors take a row a thread (32^4, nb 1, 0.4
+// GB: 82 us, 170 with 48 rows; nb 8 557 us with 48).
+constexpr int IB_THREADS = 192;
+constexpr int ib_rows(int nb) { return nb <= 4 ? 192 : 48; }
+template <int ROWS>
 __global__ __launch_bounds__(IB_THREADS) void k_import_basis(
     const cplx<double>* __restrict__ src, int nb, int Vf, int Ef, size_t rows,
     const int* __restrict__ blk_fine, cplx<double>* __restrict__ dst) {
   extern __shared__ unsigned char smem_raw[];
-  cplx<double>* s_t = reinterpret_cast<cplx<double>*>(smem_raw);  // [IB_ROWS][nb + 1]
-  const int r = threadIdx.x % IB_ROWS;
+  cplx<double>* s_t = reinterpret_cast<cplx<double>*>(smem_raw);  // [ROWS][nb + 1]
+  const int r = threadIdx.x % ROWS;
   const size_t vec = (size_t)Vf * Ef;
-  for (size_t q0 = (size_t)blockIdx.x * IB_ROWS; q0 < rows; q0 += (size_t)gridDim.x * IB_ROWS) {
-    const int n = (int)(rows - q0 < (size_t)IB_ROWS ? rows - q0 : (size_t)IB_ROWS);
+  for (size_t q0 = (size_t)blockIdx.x * ROWS; q0 < rows; q0 += (size_t)gridDim.x * ROWS) {
+    const int n = (int)(rows - q0 < (size_t)ROWS ? rows - q0 : (size_t)ROWS);
     if (r < n) {
       const size_t q = q0 + r;
       const int e = (int)(q % Ef);
       const cplx<double>* p = src + (size_t)blk_fine[q / Ef] * Ef + e;
 #pragma unroll 4
-      for (int i = threadIdx.x / IB_ROWS; i < nb; i += IB_THREADS / IB_ROWS)
+      for (int i = threadIdx.x / ROWS; i < nb; i += IB_THREADS / ROWS)
         s_t[r * (nb + 1) + i] = p[i * vec];
     }
     __syncthreads();
@@ -1199,8 +1202,10 @@ int mgc_aggregation_set_basis(mgc_aggregation* a, const void* basis_f64, void* s
     MGC_CHECK(a && basis_f64, MGC_ERR_ARG, "null argument");
     const size_t rows = (size_t)a->Vf * a->Ef;
     hipStream_t s = as_stream(stream);
-    k_import_basis<<<tile_grid((rows + IB_ROWS - 1) / IB_ROWS), IB_THREADS,
-                     (size_t)IB_ROWS * (a->nb + 1) * sizeof(cplx<double>), s>>>(
+    const int per = ib_rows(a->nb);
+    auto k = per == 48 ? k_import_basis<48> : k_import_basis<192>;
+    k<<<tile_grid((rows + per - 1) / per), IB_THREADS,
+        (size_t)per * (a->nb + 1) * sizeof(cplx<double>), s>>>(
         (const cplx<double>*)basis_f64, a->nb, a->Vf, a->Ef, rows, a->blk_fine, a->basis64);
     MGC_LAUNCH_CHECK();
     a->basis_set = true;

@@ -1,7 +1,7 @@
-"""Exact round trips through the tiled layout conversions: links (whole matrices up
-to N = 48, 32 x 32 tiles above; both external layouts) and basis (48 panel rows a
-tile), at sizes with partial tiles.  Values are moved, not computed: equality bit for bit (FP32 operators:
-equality with the rounded input)."""
+"""Exact round trips through the tiled layout conversions: links (whole matrices or
+32 x 32 tiles by N; both external layouts) and basis (48 or 192 panel rows a tile), at
+sizes with partial tiles.  Values are moved, not computed: equality bit for bit (FP32
+operators: equality with the rounded input)."""
 import numpy as np
 import pytest
 
@@ -53,6 +53,9 @@ def test_reconstructed_links(gpu, N, disp_have):
 
 
 @pytest.mark.parametrize("fd,blk,nb,Ef", [((2, 3, 1, 1), (1, 3, 1, 1), 1, 2),
+                                          ((6, 3, 3, 3), (3, 3, 1, 3), 3, 26),
+                                          ((4, 4, 2, 2), (2, 2, 2, 1), 4, 12),
+                                          ((4, 4, 2, 2), (2, 2, 2, 1), 5, 12),
                                           ((4, 4, 2, 2), (2, 2, 2, 1), 17, 12),
                                           ((6, 3, 3, 3), (3, 3, 3, 3), 33, 26),
                                           ((4, 2, 2, 2), (2, 2, 1, 2), 64, 12)])

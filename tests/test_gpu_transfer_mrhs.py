@@ -1,9 +1,9 @@
 """Project and promote of several right-hand sides (the matrix-core form, and the
-vector form in chunks of four where the dispatch keeps it) at the edges of its tiles: basis widths around multiples of 16 and 4 (odd ones among
-them), 16-rhs column tiles with remainders, blocks whose site count is no
-multiple of a wavefront's four or sixteen sites, fields of a coarse level
-(element counts other than 12), masks, panels split over workgroups, and FP32
-fields at an address that is no multiple of 16 bytes.
+vector form in chunks of four where the dispatch keeps it) at the edges of its tiles:
+basis widths around multiples of 16 and 4 (odd ones among them), 16-rhs column tiles
+with remainders, blocks whose site count is no multiple of a wavefront's four or sixteen
+sites, fields of a coarse level (element counts other than 12), masks, panels split over
+workgroups, and FP32 fields at an address that is no multiple of 16 bytes.
 
 Tolerances as in test_gpu_aggregation.py: relative L2 1e-13 in FP64 and 2e-6 in
 FP32, where basis and inputs are rounded to 2^-24 and the sums are FP32.
