@@ -436,9 +436,8 @@ void with_shape(int n, bool vec, bool fast, F&& f) {
   else f(N, std::false_type{}, std::false_type{});
 }
 
-template <typename R>
 bool aligned_fine(const mgc_aggregation* a, const void* fine) {
-  return a->Ef == 12 && (sizeof(R) == 8 || (uintptr_t)fine % 16 == 0);
+  return a->Ef == 12 && (uintptr_t)fine % 16 == 0;
 }
 
 }  // namespace
@@ -448,7 +447,7 @@ void project_mfma(const mgc_aggregation* a, const cplx<R>* U, const cplx<R>* in,
                   cplx<R>* part, int nrhs, int S, int kind, int point, hipStream_t s) {
   // VEC: each lane's MT entries are one run (and 16-byte aligned in FP32 when MT is even)
   const int mt = (a->nb + 15) / 16;
-  with_shape<4>(mt, a->nb % mt == 0, aligned_fine<R>(a, in), [&](auto MT, auto VEC, auto FAST) {
+  with_shape<4>(mt, a->nb % mt == 0, aligned_fine(a, in), [&](auto MT, auto VEC, auto FAST) {
     if constexpr (MT() > 1 || VEC())  // one entry a lane is always a run
       project_launch<R, MT(), VEC(), FAST()>(a, U, in, out, part, nrhs, S, kind, point, s);
   });
@@ -458,7 +457,7 @@ template <typename R>
 void promote_mfma(const mgc_aggregation* a, const cplx<R>* U, const cplx<R>* in, cplx<R>* out,
                   int nrhs, hipStream_t s) {
   // VEC: pairs of entries neither straddle nb nor (in FP32) a 16-byte boundary
-  with_shape<8>((a->nb + 7) / 8, a->nb % 2 == 0, aligned_fine<R>(a, out),
+  with_shape<8>((a->nb + 7) / 8, a->nb % 2 == 0, aligned_fine(a, out),
                 [&](auto KP, auto VEC, auto FAST) {
                   promote_launch<R, KP(), VEC(), FAST()>(a, U, in, out, nrhs, s);
                 });

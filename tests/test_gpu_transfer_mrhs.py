@@ -3,7 +3,7 @@ vector form in chunks of four where the dispatch keeps it) at the edges of its t
 basis widths around multiples of 16 and 4 (odd ones among them), 16-rhs column tiles
 with remainders, blocks whose site count is no multiple of a wavefront's four or sixteen
 sites, fields of a coarse level (element counts other than 12), masks, panels split over
-workgroups, and FP32 fields at an address that is no multiple of 16 bytes.
+workgroups, and fields at an address that is no multiple of 16 bytes.
 
 Tolerances as in test_gpu_aggregation.py: relative L2 1e-13 in FP64 and 2e-6 in
 FP32, where basis and inputs are rounded to 2^-24 and the sums are FP32.
@@ -66,23 +66,25 @@ def test_transfers_match_oracle(gpu, fd, blk, nb, Ef, nrhs, prec):
         ref_c.append(oracle.project_ef(fd, blk, nb, Ef, B, f[:, r].astype(np.complex128)))
         ref_f.append(oracle.promote_ef(fd, blk, nb, Ef, B, c[:, r].astype(np.complex128)))
     ref_c, ref_f = np.stack(ref_c, 1), np.stack(ref_f, 1)
-    for shift in (0, 1):  # the fields one complex number into their buffers
-        pad = np.zeros(shift, dt)
-        df = gpu.DeviceBuffer.from_numpy(np.concatenate([pad, f.ravel()]))
-        dc = gpu.DeviceBuffer.from_numpy(np.concatenate([pad, c.ravel()]))
+    real = np.float64 if prec == 0 else np.float32
+    for shift in (0, 8):  # the fields eight bytes into their buffers
+        k = shift // np.dtype(real).itemsize
+        pad = np.zeros(k, real)
+        df = gpu.DeviceBuffer.from_numpy(np.concatenate([pad, f.ravel().view(real)]))
+        dc = gpu.DeviceBuffer.from_numpy(np.concatenate([pad, c.ravel().view(real)]))
         oc = gpu.DeviceBuffer(Vc * nrhs * 2 * nb * sz)
-        of = gpu.DeviceBuffer((f.size + 2 * shift) * sz)
+        of = gpu.DeviceBuffer(f.size * sz + 2 * shift)
         of.zero()
-        agg.project(df.ptr + shift * sz, oc, prec, nrhs)
-        agg.promote(dc.ptr + shift * sz, of.ptr + shift * sz, prec, nrhs)
+        agg.project(df.ptr + shift, oc, prec, nrhs)
+        agg.promote(dc.ptr + shift, of.ptr + shift, prec, nrhs)
         gpu.synchronize()
         got_c = oc.to_numpy(dt, ref_c.shape)
-        raw = of.to_numpy(dt, (f.size + 2 * shift,))
-        got_f = raw[shift:shift + f.size].reshape(ref_f.shape)
+        raw = of.to_numpy(real, (2 * f.size + 2 * k,))
+        got_f = raw[k:k + 2 * f.size].view(dt).reshape(ref_f.shape)
         for r in range(nrhs):
             assert rel(ref_c[:, r], got_c[:, r].astype(np.complex128)) < tol, (shift, r)
             assert rel(ref_f[:, r], got_f[:, r].astype(np.complex128)) < tol, (shift, r)
-        assert not raw[:shift].any() and not raw[shift + f.size:].any()
+        assert not raw[:k].any() and not raw[k + 2 * f.size:].any()
 
 
 @pytest.mark.parametrize("prec", [0, 1])
