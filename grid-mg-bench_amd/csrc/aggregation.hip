@@ -943,8 +943,9 @@ static void check_agg(const mgc_aggregation* a) {
   MGC_CHECK(a->basis_set, MGC_ERR_STATE, "basis not set");
 }
 
-// FP64 promote takes at most 56 basis vectors, for one rhs (64 KB of LDS with
-// the four-lane tile) and for several alike
+// FP64 promote takes at most 56 basis vectors: the vector form's tile of four rhs and
+// 64 rows holds no more in 64 KB, (8 + 65) nb entries of 16 bytes.  The matrix form has
+// no such limit; the call has one for every number of rhs.
 static bool promote_nb_ok(int prec, int nb) { return prec != MGC_F64 || nb <= 56; }
 static const char* const PROMOTE_NB_MSG = "promote: nbasis too large for the LDS tile";
 
@@ -1078,9 +1079,10 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
 #define PROMOTE_R(R, RCT, LPR, T, basis)                                                      \
   k_promote<R, RCT, LPR, T><<<grid, 256, sh, s>>>(basis, (const cplx<R>*)in, (cplx<R>*)out,   \
                                                   a->blk_fine, nb, a->Vb, a->Ef, nrhs, rows_per)
-#define PROMOTE_T(R, LPR, T, basis)          \
-  if (rct == 1) PROMOTE_R(R, 1, LPR, T, basis); \
-  else PROMOTE_R(R, 4, LPR, T, basis)
+// (four lanes in FP32 are nb 60 up, which several rhs take in the matrix form)
+#define PROMOTE_T(R, LPR, T, basis)                                                           \
+  if (rct == 1) PROMOTE_R(R, 1, LPR, T, basis);                                               \
+  else if constexpr (sizeof(R) == 8 || LPR < 4) PROMOTE_R(R, 4, LPR, T, basis)
 #define PROMOTE(R, LPR, basis)                           \
   switch (tpt) {                                         \
     case 2: PROMOTE_T(R, LPR, 2, basis); break;          \
