@@ -130,7 +130,14 @@ CO_CASES = [((8, 8, 8, 8), (4, 4, 4, 4), 12),   # the reference's CPU case: 8^4 
             ((4, 4, 2, 2), (4, 2, 2, 2), 8),    # coarse extents 1 and 2
             ((4, 4, 4, 4), (2, 2, 2, 2), 16),
             ((8, 8, 8, 8), (4, 4, 4, 4), 20),   # the reference's default nbasis 40
-            ((4, 4, 4, 4), (2, 2, 2, 2), 30)]
+            ((4, 4, 4, 4), (2, 2, 2, 2), 30),
+            ((4, 4, 4, 4), (2, 2, 2, 2), 32),   # the widest basis, no padded rows or columns
+            ((4, 4, 4, 4), (2, 2, 2, 2), 24),
+            ((3, 3, 6, 3), (3, 3, 3, 3), 12),   # 81 and 27 sites: no multiple of a stage's four
+            ((6, 3, 3, 3), (3, 3, 3, 3), 24),   # ... or two
+            ((6, 4, 4, 2), (3, 1, 2, 1), 16),   # block extents of 1, faces of 2 and 6 sites
+            ((6, 2, 4, 3), (3, 1, 2, 1), 32),
+            ((4, 3, 2, 2), (1, 1, 1, 1), 4)]    # one site a block
 
 
 @pytest.fixture(params=[1, 0], ids=["mfma", "vector"])
