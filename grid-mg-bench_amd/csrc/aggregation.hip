@@ -991,10 +991,11 @@ void agg_transfer(mgc_aggregation* a, const void* in, void* out, int prec, int n
     const bool few = nrhs <= 4 && S > 1 && rows < 768 && (f64 || nrhs < 4);
     // Project's chains of additions are no longer than the vector form's
     // (k_project_mfma) on blocks of eight Dirac sites or more, and in a split panel of
-    // longer records from 192 rows a workgroup up (FP64, nb 32, 64 elements: 64 rows
-    // 1.05 times its error).
-    const bool short_chains =
-        a->Vb >= 8 && rows >= 96 && (S == 1 || a->Ef == 12 || rows_per >= 192);
+    // longer records from 192 rows a workgroup up (error at 64 rows and 64 elements
+    // against the vector form's: FP64 nb 32 1.07, FP32 nb 48 and 64 1.03, 1.04; FP32 to
+    // nb 32, which has twice the groups there, 0.89 to 0.99).
+    const bool short_chains = a->Vb >= 8 && rows >= 96 &&
+                              (S == 1 || a->Ef == 12 || rows_per >= 192 || (!f64 && nb <= 32));
     matrix = matrix && short_chains && !thin && !few;
   } else {
     // - nb 1 to 4: 3^4 blocks (sites no multiple of the 16 columns) 0.9 to 1.9 at any
