@@ -330,9 +330,9 @@ __global__ __launch_bounds__(4 * (NB / TC) * (NB / TC)) void k_coarsen(
 // FP32 16x16x4 form's 4(l/16) + r).
 //
 // What bounds it: the products (412 GFLOP at 32^4, 4^4 blocks, nb 32: 5.7 ms at
-// the FP64 matrix rate) and, for the self point, the gathers of W: the panel
-// comes from beyond L2 three times (20 GB).  The workgroups of a CU overlap the
-// two, so a stage is sized for three of them (38 KB of LDS: two sites at nb >
+// the FP64 matrix rate) and the gathers of W: the self point reads 43 GB from beyond
+// L2, over six times the panel, at 4.7 TB/s, the faces 12 GB (55 GB in all; 51 in one
+// kernel with two workgroups a CU).  The workgroups of a CU overlap the two, so a stage is sized for three of them (38 KB of LDS: two sites at nb >
 // 16, four below; up to 168 registers a lane).  For the registers a W item is
 // one spin of one chirality (two lanes per column), the link, the same for a
 // whole wavefront, is read into scalar registers, and the faces and the self

@@ -622,9 +622,11 @@ __global__ __launch_bounds__(256) void k_wilson_lds(const cplx<R>* __restrict__ 
 // k_wilson_lds.
 // Which site, rhs and chunk a thread copies is the same in every stage: the
 // divisions by nrhs are done once and their results kept, one register a chunk,
-// and the neighbour sites are kept as 32-bit chunk indexes too.  With the divisions in each stage the
-// integer multiplies took twice the time of the FP32 arithmetic: 12 rhs at 32^4
-// 1.42 ms.
+// and the neighbour sites are kept as 32-bit chunk indexes too.  With the divisions in
+// each stage the integer multiplies took twice the time of the FP32 arithmetic: 12 rhs
+// at 32^4 1.42 ms, now 1.17.
+// What bounds it: 4.32 GB read at that size, 2.4 times the 1.81 it must, and 1.21
+// written: 4.7 TB/s, a copy's rate, with the vector units about 70% busy.
 template <typename R, int LPT, bool DAG>
 __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U,
                                                    const cplx<R>* __restrict__ diag,
@@ -769,8 +771,9 @@ __global__ __launch_bounds__(256) void k_wilson_pf(const cplx<R>* __restrict__ U
 // self first, then 0..7; each stage's records are staged in LDS (each read by
 // the three threads of the site), the next stage's loads issued before its
 // arithmetic.
-// What bounds it: HBM traffic is the algorithmic one (48^4 FP64: 6.8 GB read, 1.0
-// written); the rest is latency, so the loads that do not depend on others are
+// What bounds it: it reads 1.9 times what it must, since neighbour spinors and
+// backward links come again from beyond L2 (48^4 FP64: 13.5 GB of 7.1, and 1.02
+// written: 7.0 TB/s), and latency, so the loads that do not depend on others are
 // issued together.  48^4 FP64 2.19 -> 2.08 ms, 32^4 FP32 0.233 -> 0.206, 16^4 FP32
 // 20.6 -> 13.4 us against one stage's loads at a time (neighbour sites one hop
 // ahead, clover entries during their arithmetic).  Two hops a stage: 0.257 ms at

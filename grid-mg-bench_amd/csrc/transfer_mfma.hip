@@ -14,8 +14,8 @@
 // What bounds them is HBM: the basis, V x Ef x nb entries, is read once per 16
 // right-hand sides (the vector-unit kernels read it once per four), and the
 // fine field is read or written once.  At 32^4, 4^4 blocks, nb 16, 12 rhs, FP32
-// that is 2.8 GB a direction: project 0.55 ms (5.1 TB/s; 1.45 ms in the vector
-// form), promote 0.55 ms (1.27 ms).
+// that is 2.8 GB a direction (3.24 and 2.84 measured): project 0.50 ms (1.45 ms in the
+// vector form), promote 0.59 ms (1.27 ms).
 //
 // Both kernels are instantiated for the width of the basis.  VEC: nb allows
 // vector loads of it; FAST: Ef = 12 and a fine field at a 16-byte address.
